@@ -24,9 +24,8 @@
 //
 // Mapping.  A workgroup of 4 waves owns 64 gate and 64 up rows (wave w:
 // rows 16 w .. 16 w + 15 of both, so SwiGLU is applied in registers) or 128
-// down rows (wave w: two tiles of 16) -- the three-plane gate/up GEMM twice
-// that, 32 rows of gate and of up per wave -- for one chunk of <= 16 NB
-// tokens of one expert.  Weight rows are the MFMA columns (B operand): lane (c, j)
+// down rows (wave w: two tiles of 16) for one chunk of tokens of one expert.
+// Weight rows are the MFMA columns (B operand): lane (c, j)
 // holds row c and group j (qs bytes 32 j .. 32 j + 31, sub-blocks 2j, 2j+1)
 // of every block, read as two whole 16-byte pieces of the resident expert
 // layout, so the four lanes of a row read one 64-byte line per load and
@@ -36,6 +35,25 @@
 // LDS) reads the same elements.  Per block the chunk's token planes are
 // copied global -> LDS by direct loads into one of two buffers, so block
 // b + 1 streams in while block b is contracted.
+//
+// What bounds it.  A read of the same weight lines with the same tiles and
+// no math takes 180-205 us for 71 experts' gate and up (5.7-6.6 TB/s); the
+// vector ALU (about 105 instructions per 16-row tile and block, 9 per 8
+// weights for the operand) and the matrix cores (16 cycles per 16x16x32, 32
+// per 16x16x4) need about as long and overlap only partly, so the kernel
+// lives on loads in flight and on few instructions:
+//  - the three planes of a chunk of few tokens share 16-row operands (PACK):
+//    up to 5 tokens cost 8 MFMAs per tile and block instead of 24 and a
+//    third of the LDS traffic; with that, two tiles per wave and three waves
+//    per SIMD beat four tiles and two waves (16-token step 234 against 279 us);
+//  - each weight register is refilled with block b + 2 right after its last
+//    use, so the stream runs one to two blocks ahead on two register sets
+//    (234 -> 219 us, 64 tokens 479 -> 443 us);
+//  - buffer loads: no address arithmetic on the vector ALU;
+//  - an expert with one chunk is streamed past the L2 (nontemporal).
+// gate/up of 71 / 132 / 188 experts (16 / 64 / 256 tokens): 328 -> 219, 587 ->
+// 443, 1032 -> 925 us; the down of 16 / 256 tokens 151 -> 122, 517 -> 479 us;
+// one plane, 512 tokens: gate/up 994 -> 906, down 522 -> 499 us.
 #include "fdm_internal.h"
 #include "planes_device.h"
 
@@ -48,15 +66,15 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kQWaves = 4;            // waves per workgroup
 constexpr int kQRowB = kQK * 2;       // LDS token row: one block of fp16 (512 B)
-// Weight tiles of 16 rows per wave (TL): a gate/up GEMM holds TL / 2 tiles of
-// gate and as many of up (SwiGLU pairs tile t with tile t + TL / 2), a down
-// GEMM TL tiles; every token operand read from LDS serves all of them.  Four
-// tiles for the fp32-grade gate/up (three planes: twice the weights per token
-// operand read, 252 VGPRs), two elsewhere (168 VGPRs for the three-plane down:
-// 3 waves per SIMD; 213-229 for one plane: 2 waves per SIMD, no spills).
-__host__ __device__ constexpr int qgemm_tiles(int planes, bool down) { return (planes == 3 && !down) ? 4 : 2; }
-__host__ __device__ constexpr int qgemm_rows(int tiles, bool down) {  // rows per workgroup (of gate for gate/up)
-  return (down ? 16 : 8) * tiles * kQWaves;
+constexpr int kQMaxTok = 64;          // tokens of the largest chunk
+// Weight tiles of 16 rows per wave: one of gate and one of up (SwiGLU pairs
+// them), or two of down; every token operand read from LDS serves both.
+constexpr int kQTiles = 2;
+// Waves per SIMD: 3 for three planes (168 VGPRs), 2 for one plane, whose
+// 64-token chunks hold four operand blocks of accumulators.
+__host__ __device__ constexpr int qgemm_waves(int planes) { return planes == 3 ? 3 : 2; }
+__host__ __device__ constexpr int qgemm_rows(bool down) {  // rows per workgroup (of gate for gate/up)
+  return (down ? 16 : 8) * kQTiles * kQWaves;
 }
 
 // One lane's share of one block of one weight row (resident expert layout):
@@ -64,31 +82,6 @@ __host__ __device__ constexpr int qgemm_rows(int tiles, bool down) {  // rows pe
 struct QLane {
   u32x4 q0, q1, hdr;
 };
-
-// A block's q0 (and q1) pieces of a row pair (gate / up) or quad (down) fill
-// whole 128-byte lines of the resident layout, read once per chunk of the
-// expert.  Odd blocks are read with the nontemporal policy, even ones with
-// the default policy: measured a little faster than either policy for every
-// block (the default lines stay in the L2 for the expert's other chunks,
-// the streamed half leaves room).
-template <bool DOWN, bool LAST>
-__device__ __forceinline__ QLane qlane_load(const uint8_t* mat, int row, int block, int j) {
-  constexpr int N = DOWN ? kRelDnPieces : kRelGuPieces;
-  const uint8_t* st = rel_step<DOWN>(mat, row, block);
-  const int L0 = rel_piece<DOWN>(row, block, 0);
-  const u32x4* p0 = reinterpret_cast<const u32x4*>(st + 16 * (L0 + j));
-  const u32x4* p1 = reinterpret_cast<const u32x4*>(st + 16 * N + 16 * (L0 + j));
-  QLane r;
-  if (LAST) {
-    r.q0 = __builtin_nontemporal_load(p0);
-    r.q1 = __builtin_nontemporal_load(p1);
-  } else {
-    r.q0 = *p0;
-    r.q1 = *p1;
-  }
-  r.hdr = *reinterpret_cast<const u32x4*>(st + 32 * N + 4 * L0);
-  return r;
-}
 
 // fp16 halves of sc * q for the two q held in bits 0-3 (MASK 0x000F000F)
 // of the halves of w, the rest of w arbitrary: 0x6400 | q is the half
@@ -170,12 +163,30 @@ __device__ __forceinline__ f32x4 mfma_f(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// One 16-byte direct global -> LDS load per lane (lane i writes lds_dst + 16 i).
-__device__ __forceinline__ void lds_dma16(const void* gsrc, void* lds_dst) {
-  __builtin_amdgcn_global_load_lds(gsrc, lds_dst, 16, 0, 0);
+// Buffer accesses: a uniform 128-bit descriptor, a constant 32-bit offset per
+// lane and a uniform one per block, so no address arithmetic runs on the
+// vector ALU and no lane holds a 64-bit address.
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+__device__ __forceinline__ rsrc_t make_rsrc(const void* p, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000);
+}
+constexpr int kCacheNt = 2;  // the nontemporal policy bit of a buffer access
+template <int POLICY>
+__device__ __forceinline__ u32x4 buf_load16(rsrc_t r, uint32_t lane_off, uint32_t off) {
+  return __builtin_amdgcn_raw_buffer_load_b128(r, (int)lane_off, (int)off, POLICY);
 }
 
-__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// One 16-byte direct global -> LDS load per lane (lane i writes lds_dst + 16 i).
+__device__ __forceinline__ void lds_dma16(rsrc_t r, uint32_t lane_off, uint32_t off, void* lds_dst) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds_dst, 16, (int)lane_off,
+                                           (int)off, 0, 0);
+}
+
+// waits until at most N of the wave's loads are in flight
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
 
 }  // namespace
 
@@ -219,72 +230,115 @@ __global__ __launch_bounds__(256) void k_xplanes(const float* __restrict__ x, si
 }
 
 // ---- the grouped GEMM ------------------------------------------------------------------
-template <int P, int NB, bool DOWN, int TL>
-__device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, uint8_t* lds1, int* rows, int chunk, int rg) {
+// One chunk (n tokens) of one expert, one row group.  The token operand has
+// PK * 16 NB rows in LDS: with PACK = false row (p, r) is plane p of token r
+// and a token block's PK planes accumulate into one register set; with PACK
+// = true (PK = 1) row r is plane r / n of token r % n, so the three planes
+// of up to 5 (NB = 1) or 10 (NB = 2) tokens share the 16-row operands that
+// padding would otherwise fill, and are added up once after the last block.
+// NT: the expert has one chunk, its weights are read once and streamed past
+// the L2.
+template <int P, int PK, int NB, bool PACK, bool DOWN, bool NT>
+__device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, uint8_t* lds1, int* rows, const int4 ck,
+                                           int rg) {
+  static_assert(PACK ? PK == 1 && P == 3 : PK == P, "packed rows carry one plane each");
+  constexpr int TL = kQTiles;
   constexpr int KD = DOWN ? kFfn : kHidden;  // contraction length
   constexpr int NBLK = KD / kQK;             // 8 or 28 (even)
-  constexpr int NT = 16 * NB;                // token rows per buffer and plane
-  constexpr int BUF = P * NT * kQRowB;       // bytes per buffer
-  constexpr int ROUNDS = P * NT / (2 * kQWaves);  // direct loads per wave per block (2 rows each)
-  static_assert(ROUNDS * 2 * kQWaves == P * NT, "the direct loads tile the buffer");
-  const int4 ck = g.chunks[chunk];
+  constexpr int NT16 = 16 * NB;              // operand rows per plane slot
+  constexpr int NTOK = PACK ? NT16 / 3 : NT16;
+  constexpr int NBX = (NTOK + 15) / 16;      // 16-row blocks that hold plane 0 rows
+  constexpr int ROUNDS = PK * NT16 / (2 * kQWaves);  // direct loads per wave per block (2 rows each)
+  static_assert(ROUNDS * 2 * kQWaves == PK * NT16, "the direct loads tile the buffer");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c16 = lane & 15, j = lane >> 4;
   const int n = ck.z;
   const bool shared = ck.x < 0;
   const int P0 = g.T * g.K;
-  int* rin = rows;          // input row of chunk token t (activation plane row)
-  int* rout = rows + NT;    // output row
-  if (threadIdx.x < NT) {
-    const int t = min((int)threadIdx.x, n - 1);  // pad rows repeat the last token
+  int* rin = rows;              // input row of chunk token t (activation plane row)
+  int* rout = rows + kQMaxTok;  // output row
+  if (threadIdx.x < n) {
+    const int t = threadIdx.x;
     const int orow = shared ? P0 + ck.y + t : ck.y + t;
-    rout[threadIdx.x] = orow;
-    rin[threadIdx.x] = DOWN ? orow : (shared ? ck.y + t : g.pair_tok[ck.y + t]);
+    rout[t] = orow;
+    rin[t] = DOWN ? orow : (shared ? ck.y + t : g.pair_tok[ck.y + t]);
   }
-  __syncthreads();
+  // weight addresses: a uniform base per block and constant lane offsets
   const uint8_t* blob = shared ? g.shared : g.experts + (size_t)ck.x * g.expert_size;
-  constexpr int ROWS = qgemm_rows(TL, DOWN);
-  const uint8_t* mat[TL];
+  const uint8_t* mat = blob + (DOWN ? 2 * (size_t)kGateBytes : 0);
+  constexpr int ROWS = qgemm_rows(DOWN);
+  uint32_t qoff[TL], hoff[TL];
   int row[TL];
 #pragma unroll
   for (int t = 0; t < TL; ++t) {
-    if (DOWN) {
-      mat[t] = blob + 2 * (size_t)kGateBytes;
-      row[t] = rg * ROWS + 16 * TL * wave + 16 * t + c16;
-    } else {
-      // tiles 0 .. TL/2 - 1: gate rows, TL/2 .. TL - 1: the same rows of up
-      mat[t] = blob + (t < TL / 2 ? 0 : (size_t)kGateBytes);
-      row[t] = rg * ROWS + 8 * TL * wave + 16 * (t % (TL / 2)) + c16;
-    }
+    // gate/up: tiles 0 .. TL/2 - 1 gate rows, TL/2 .. TL - 1 the same rows of up
+    row[t] = DOWN ? rg * ROWS + 16 * TL * wave + 16 * t + c16 : rg * ROWS + 8 * TL * wave + 16 * (t % (TL / 2)) + c16;
+    const uint32_t base = (uint32_t)(rel_step<DOWN>(nullptr, row[t], 0) - (const uint8_t*)nullptr) +
+                          (!DOWN && t >= TL / 2 ? (uint32_t)kGateBytes : 0u);
+    const int L0 = rel_piece<DOWN>(row[t], 0, 0);
+    qoff[t] = base + 16u * (uint32_t)(L0 + j);
+    hoff[t] = base + 32u * (DOWN ? kRelDnPieces : kRelGuPieces) + 4u * (uint32_t)L0;
   }
-  // direct-load sources: round k of wave w fills LDS rows 2 (w + 8 k), +1 of
-  // the buffer (row rho = plane * NT + token t); lane i: row rho0 + i / 32,
-  // slot i % 32 holds piece (i % 32) ^ (t & 7) of that row's block.  The
+  const rsrc_t wr = make_rsrc(mat, (DOWN ? 1 : 2) * (size_t)kGateBytes);
+  auto load_hdr = [&](QLane (&w)[TL], int b) {
+    const uint32_t st = (uint32_t)(rel_step<DOWN>(nullptr, 0, b) - (const uint8_t*)nullptr);
+#pragma unroll
+    for (int t = 0; t < TL; ++t) w[t].hdr = buf_load16<0>(wr, hoff[t], st + 4 * (uint32_t)rel_piece<DOWN>(0, b, 0));
+  };
+  auto load_q = [&](QLane (&w)[TL], int b, int half) {
+    const uint32_t st = (uint32_t)(rel_step<DOWN>(nullptr, 0, b) - (const uint8_t*)nullptr) +
+                        16 * (uint32_t)(rel_piece<DOWN>(0, b, 0) + half * (DOWN ? kRelDnPieces : kRelGuPieces));
+#pragma unroll
+    for (int t = 0; t < TL; ++t) (half ? w[t].q1 : w[t].q0) = buf_load16<NT ? kCacheNt : 0>(wr, qoff[t], st);
+  };
+  QLane wa[TL], wb[TL];
+  load_hdr(wa, 0);
+  load_q(wa, 0, 0);
+  load_q(wa, 0, 1);
+  __syncthreads();  // rin, rout
+  // operand row r of plane slot p -> (plane, token)
+  auto row_token = [&](int r, int p, int& plane) {
+    if (PACK) {
+      r = min(r, 3 * n - 1);
+      plane = (r >= n) + (r >= 2 * n);
+      return r - plane * n;
+    }
+    plane = p;
+    return min(r, n - 1);  // pad rows repeat the last token
+  };
+  // direct-load sources: round k of wave w fills LDS rows 2 (w + 4 k), +1 of
+  // the buffer (row rho = slot * NT16 + r); lane i: row rho0 + i / 32,
+  // slot i % 32 holds piece (i % 32) ^ (r & 7) of that row's block.  The
   // token operand's 16-byte reads (lane (c16, j): row c16, piece
   // (8 j + m) ^ (c16 & 7)) are then free of bank conflicts; an XOR with all
   // four bits of c16 measured twice the cycles per read (2-way conflicts).
+  const rsrc_t pr = make_rsrc(g.xp, 2 * P * g.plane);
   uint32_t src[ROUNDS];
 #pragma unroll
   for (int k = 0; k < ROUNDS; ++k) {
     const int rho = 2 * (wave + kQWaves * k) + (lane >> 5);
-    const int p = rho / NT, t = rho - p * NT;
-    const uint32_t piece = (uint32_t)((lane & 31) ^ (t & 7));
-    src[k] = (uint32_t)((size_t)rin[t] * KD) + 8u * piece;  // element offset inside plane p
+    const int p = rho / NT16, r = rho - p * NT16;
+    int plane;
+    const int t = row_token(r, p, plane);
+    const uint32_t piece = (uint32_t)((lane & 31) ^ (r & 7));
+    src[k] = 2u * ((uint32_t)plane * (uint32_t)g.plane + (uint32_t)(rin[t] * KD) + 8u * piece);  // byte offset
   }
   auto dma = [&](int b, int buf) {
     uint8_t* base = buf ? lds1 : lds0;
 #pragma unroll
-    for (int k = 0; k < ROUNDS; ++k) {
-      const int rho0 = 2 * (wave + kQWaves * k);
-      const int p = rho0 / NT;
-      lds_dma16(g.xp + (size_t)p * g.plane + src[k] + (size_t)b * kQK, base + rho0 * kQRowB);
-    }
+    for (int k = 0; k < ROUNDS; ++k) lds_dma16(pr, src[k], (uint32_t)b * (2 * kQK), base + 2 * (wave + kQWaves * k) * kQRowB);
   };
   const Q4KScaleSel sel = q4k_scale_sel(j);
-  // corr operand A: token c16 of block nb, sub-blocks 2j and 2j+1 of block b
-  auto load_xs = [&](int b, int nb) {
-    const float2 v = *reinterpret_cast<const float2*>(g.xs + (size_t)rin[16 * nb + c16] * (KD / 32) + 8 * b + 2 * j);
-    return v;
+  // corr operand A: plane 0 row c16 of block nb, sub-blocks 2j and 2j+1 of block b
+  uint32_t xoff[NBX];
+#pragma unroll
+  for (int nb = 0; nb < NBX; ++nb) xoff[nb] = (uint32_t)(rin[min(16 * nb + c16, n - 1)] * (KD / 32) + 2 * j);
+  auto load_xs = [&](float2 (&v)[NBX], int b) {
+#pragma unroll
+    for (int nb = 0; nb < NBX; ++nb) {
+      v[nb] = *reinterpret_cast<const float2*>(g.xs + 8 * b + xoff[nb]);
+      if (PACK && 16 * nb + c16 >= n) v[nb] = float2{0.0f, 0.0f};  // a row of another plane
+    }
   };
   f32x4 acc[TL][NB];
 #pragma unroll
@@ -293,12 +347,21 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
     for (int nb = 0; nb < NB; ++nb) acc[tt][nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   // One block: the token operands of an MFMA step are read from LDS once and
-  // serve every tile, whose B operands are built per step.
-  auto block = [&](int buf, const QLane (&w)[TL], const float2 (&xsv)[NB]) {
+  // serve every tile, whose B operands are built per step.  With refill, each
+  // weight register is loaded with block b + 2 right after its last use: the
+  // weight stream runs one to two blocks ahead on two register sets.
+  auto block = [&](int buf, QLane (&w)[TL], const float2 (&xsv)[NBX], bool refill, int b) {
     const uint8_t* base = buf ? lds1 : lds0;
     QScale sc[TL];
 #pragma unroll
-    for (int t = 0; t < TL; ++t) sc[t] = qscale(w[t].hdr, sel);
+    for (int t = 0; t < TL; ++t) {
+      sc[t] = qscale(w[t].hdr, sel);
+      // every constant is in a register of its own here: the header's are free
+      asm volatile("" : "+v"(sc[t].d), "+v"(sc[t].k_lo), "+v"(sc[t].k_hi), "+v"(sc[t].bc_lo), "+v"(sc[t].bc_hi));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (refill) load_hdr(w, b + 2);
+    __builtin_amdgcn_sched_barrier(0);
     f32x4 C[TL][NB];
 #pragma unroll
     for (int t = 0; t < TL; ++t)
@@ -307,48 +370,29 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       const int i0 = 2 * (m & 1);
-      if constexpr (TL == 2) {
-        // both tiles' B operands first, then each token operand read once
-        // and used by both
-        const u32x4& qa = m < 2 ? w[0].q0 : w[0].q1;
-        const u32x4& qb = m < 2 ? w[1].q0 : w[1].q1;
-        const BPair B0 = build_b(qa[i0], qa[i0 + 1], sc[0].k_lo, sc[0].k_hi);
-        const BPair B1 = build_b(qb[i0], qb[i0 + 1], sc[1].k_lo, sc[1].k_hi);
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-          for (int p = 0; p < P; ++p) {
-            const uint8_t* r = base + (p * NT + 16 * nb + c16) * kQRowB;
-            const f16x8 alo = *reinterpret_cast<const f16x8*>(r + 16 * ((8 * j + m) ^ (c16 & 7)));
-            const f16x8 ahi = *reinterpret_cast<const f16x8*>(r + 16 * ((8 * j + m + 4) ^ (c16 & 7)));
-            C[0][nb] = mfma_h(alo, B0.lo, C[0][nb]);
-            C[1][nb] = mfma_h(alo, B1.lo, C[1][nb]);
-            C[0][nb] = mfma_h(ahi, B0.hi, C[0][nb]);
-            C[1][nb] = mfma_h(ahi, B1.hi, C[1][nb]);
-          }
-        }
-        continue;
-      }
-      f16x8 alo[NB][P], ahi[NB][P];
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-          const uint8_t* r = base + (p * NT + 16 * nb + c16) * kQRowB;
-          alo[nb][p] = *reinterpret_cast<const f16x8*>(r + 16 * ((8 * j + m) ^ (c16 & 7)));
-          ahi[nb][p] = *reinterpret_cast<const f16x8*>(r + 16 * ((8 * j + m + 4) ^ (c16 & 7)));
-        }
+      BPair B[TL];
 #pragma unroll
       for (int t = 0; t < TL; ++t) {
-        const u32x4& qa = m < 2 ? w[t].q0 : w[t].q1;
-        const BPair B = build_b(qa[i0], qa[i0 + 1], sc[t].k_lo, sc[t].k_hi);
+        const u32x4& q = m < 2 ? w[t].q0 : w[t].q1;
+        B[t] = build_b(q[i0], q[i0 + 1], sc[t].k_lo, sc[t].k_hi);
+      }
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
+      for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-          for (int p = 0; p < P; ++p) {
-            C[t][nb] = mfma_h(alo[nb][p], B.lo, C[t][nb]);
-            C[t][nb] = mfma_h(ahi[nb][p], B.hi, C[t][nb]);
-          }
+        for (int p = 0; p < PK; ++p) {
+          const uint8_t* r = base + (p * NT16 + 16 * nb + c16) * kQRowB;
+          const f16x8 alo = *reinterpret_cast<const f16x8*>(r + 16 * ((8 * j + m) ^ (c16 & 7)));
+          const f16x8 ahi = *reinterpret_cast<const f16x8*>(r + 16 * ((8 * j + m + 4) ^ (c16 & 7)));
+#pragma unroll
+          for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(alo, B[t].lo, C[t][nb]);
+#pragma unroll
+          for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(ahi, B[t].hi, C[t][nb]);
+        }
+      }
+      if (refill && (m & 1)) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_q(w, b + 2, m >> 1);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
 #pragma unroll
@@ -358,78 +402,98 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
         f32x4 a = acc[t][nb];
 #pragma unroll
         for (int i = 0; i < 4; ++i) a[i] = fmaf(sc[t].d, C[t][nb][i], a[i]);
-        a = mfma_f(xsv[nb].x, sc[t].bc_lo, a);
-        a = mfma_f(xsv[nb].y, sc[t].bc_hi, a);
+        if (nb < NBX) {
+          a = mfma_f(xsv[nb].x, sc[t].bc_lo, a);
+          a = mfma_f(xsv[nb].y, sc[t].bc_hi, a);
+        }
         acc[t][nb] = a;
       }
   };
-  auto load_w = [&](QLane (&w)[TL], int b, bool last) {
-#pragma unroll
-    for (int t = 0; t < TL; ++t)
-      w[t] = last ? qlane_load<DOWN, true>(mat[t], row[t], b, j) : qlane_load<DOWN, false>(mat[t], row[t], b, j);
-  };
 
   dma(0, 0);
-  QLane wa[TL], wb[TL];
-  load_w(wa, 0, false);
-  float2 xa[NB];
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) xa[nb] = load_xs(0, nb);
-  for (int b = 0; b < NBLK; b += 2) {
-    // even block b from buffer 0 while b + 1 lands in buffer 1, then odd
-    // block b + 1 from buffer 1 while b + 2 lands in buffer 0 (the last pair
-    // re-stages the final block into the idle buffer: branch-free, so the
-    // wait counts stay exact)
-    wait_vm();
+  float2 xa[NBX], xb[NBX];
+  load_xs(xa, 0);
+  load_hdr(wb, 1);
+  load_q(wb, 1, 0);
+  load_q(wb, 1, 1);
+  // Block b from buffer b & 1 while block b + 1 lands in the other one.  The
+  // wait before a block leaves the 3 TL youngest loads in flight (the weights
+  // of block b + 1): the loads before them, block b's weights, operands and
+  // sub-block sums, have then landed.
+  auto pair = [&](int b, bool last) {
+    wait_vm<3 * TL>();
     __syncthreads();  // block b staged by every wave; buffer 1 read by all (block b - 1)
     dma(b + 1, 1);
-    load_w(wb, b + 1, true);
-    float2 xb[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) xb[nb] = load_xs(b + 1, nb);
-    // keep the next block's loads ahead of this block's contraction (the
-    // scheduler otherwise sinks them to just before the wait, to save
-    // registers, and the stream is no longer a block ahead)
+    load_xs(xb, b + 1);
     __builtin_amdgcn_sched_barrier(0);
-    block(0, wa, xa);
-    const int b2 = min(b + 2, NBLK - 1);
-    wait_vm();
+    block(0, wa, xa, !last, b);
+    if (last)
+      wait_vm<0>();
+    else
+      wait_vm<3 * TL>();
     __syncthreads();  // block b + 1 staged; buffer 0 read by all (block b)
-    dma(b2, 0);
-    load_w(wa, b2, false);
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) xa[nb] = load_xs(b2, nb);
+    if (!last) {
+      dma(b + 2, 0);
+      load_xs(xa, b + 2);
+    }
     __builtin_amdgcn_sched_barrier(0);
-    block(1, wb, xb);
-  }
-  wait_vm();  // the re-staged copy has landed before the LDS is released
+    block(1, wb, xb, !last, b + 1);
+  };
+  for (int b = 0; b < NBLK - 2; b += 2) pair(b, false);
+  pair(NBLK - 2, true);
   // D of a 16x16 MFMA: lane (c16, j) holds row (column) c16 of the tile and
-  // tokens 4 j .. 4 j + 3 of the token block
+  // operand rows 4 j .. 4 j + 3 of the 16-row block
+  auto put = [&](int t, int tile, float gate, float up) {
+    const float e = g.xe[rin[t]];
+    if (DOWN)
+      g.out[(size_t)rout[t] * kHidden + row[tile]] = gate * e;
+    else
+      g.out[(size_t)rout[t] * kFfn + row[tile]] = silu_mul(gate * e, up * e);
+  };
+  constexpr int OT = DOWN ? TL : TL / 2;  // output tiles
+  if constexpr (!PACK) {
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
+    for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = 16 * nb + 4 * j + i;
-      if (t >= n) continue;
-      const float e = g.xe[rin[t]];
-      if (DOWN) {
-        float* o = g.out + (size_t)rout[t] * kHidden;
+      for (int i = 0; i < 4; ++i) {
+        const int t = 16 * nb + 4 * j + i;
+        if (t >= n) continue;
 #pragma unroll
-        for (int tt = 0; tt < TL; ++tt) o[row[tt]] = acc[tt][nb][i] * e;
-      } else {
-#pragma unroll
-        for (int tt = 0; tt < TL / 2; ++tt)
-          g.out[(size_t)rout[t] * kFfn + row[tt]] = silu_mul(acc[tt][nb][i] * e, acc[tt + TL / 2][nb][i] * e);
+        for (int tt = 0; tt < OT; ++tt) put(t, tt, acc[tt][nb][i], DOWN ? 0.0f : acc[DOWN ? tt : tt + TL / 2][nb][i]);
       }
+    }
+  } else {
+    // the three planes of a token lie in other lanes' rows: through a
+    // wave-private piece of buffer 0 (no longer read or written: the last
+    // block is in buffer 1), tile by tile
+    float* red = reinterpret_cast<float*>(lds0) + wave * (DOWN ? 1 : 2) * NT16 * 16;
+#pragma unroll
+    for (int tt = 0; tt < OT; ++tt) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 16 * nb + 4 * j + i;
+          red[r * 16 + c16] = acc[tt][nb][i];
+          if (!DOWN) red[(NT16 + r) * 16 + c16] = acc[DOWN ? tt : tt + TL / 2][nb][i];
+        }
+      auto sum = [&](const float* p) { return (p[2 * n * 16] + p[n * 16]) + p[0]; };
+      for (int t = j; t < n; t += 4) {
+        const float* p = red + t * 16 + c16;
+        put(t, tt, sum(p), DOWN ? 0.0f : sum(p + NT16 * 16));
+      }
+      __builtin_amdgcn_wave_barrier();  // the next tile's values overwrite these
     }
   }
 }
 
 // NB: the largest token block count of a chunk (1 for the 16-token chunks
 // of batched decode, 4 for the 64-token chunks of prefill); a chunk runs the
-// body of the fewest 16-token blocks that hold its tokens, so its weight
-// operands are built once for up to 64 tokens and no MFMA runs on an empty
-// block.  One-dimensional grid, mapped so that all the
+// body of the fewest 16-row operand blocks that hold its tokens (three planes:
+// 3 n packed rows up to 10 tokens; from 11 on the packed rows fill three
+// blocks too, and the planes of a token accumulate in registers), so its
+// weight operands are built once for up to 64 tokens and no MFMA runs on an
+// empty block.  One-dimensional grid, mapped so that all the
 // chunks of one expert that share a row group run on the same XCD, back to
 // back: workgroups are handed to the eight XCDs in turn (id % 8), so
 // id -> (xcd = id % 8, k = id / 8); XCD x owns row groups x, x + 8, ...
@@ -438,10 +502,29 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
 // (q = RG / 8), row group 8 ((k - q f) / c) + x of chunk f + (k - q f) % c.
 // An expert's weights are then read from HBM once per row group and served
 // from that XCD's L2 to its other chunks; every XCD does the same work.
+template <int P, int NB, bool DOWN, bool NT>
+__device__ __forceinline__ void qgemm_chunk(const QGemmArgs& g, uint8_t* lds0, uint8_t* lds1, int* rows, const int4 ck,
+                                            int rg) {
+  const int n = ck.z;
+  if constexpr (P == 3) {
+    if (n <= 5) return qgemm_body<3, 1, 1, true, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
+    if (n <= 10) return qgemm_body<3, 1, 2, true, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
+    return qgemm_body<3, 3, 1, false, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
+  } else {
+    if constexpr (NB == 4) {
+      if (n > 48) return qgemm_body<P, P, 4, false, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
+      if (n > 32) return qgemm_body<P, P, 3, false, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
+    }
+    if constexpr (NB >= 2) {
+      if (n > 16) return qgemm_body<P, P, 2, false, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
+    }
+    return qgemm_body<P, P, 1, false, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
+  }
+}
+
 template <int P, int NB, bool DOWN>
-__global__ __launch_bounds__(kQWaves * 64) __attribute__((amdgpu_waves_per_eu((P == 3 && DOWN) ? 3 : 2))) void k_qgemm(QGemmArgs g) {
-  constexpr int TL = qgemm_tiles(P, DOWN);
-  constexpr int RG = (DOWN ? kHidden : kFfn) / qgemm_rows(TL, DOWN);
+__global__ __launch_bounds__(kQWaves * 64) __attribute__((amdgpu_waves_per_eu(qgemm_waves(P)))) void k_qgemm(QGemmArgs g) {
+  constexpr int RG = (DOWN ? kHidden : kFfn) / qgemm_rows(DOWN);
   constexpr int Q = RG / 8;
   static_assert(Q * 8 == RG, "row groups split evenly over the XCDs");
   const int id = blockIdx.x, xcd = id & 7, k = id >> 3;
@@ -450,22 +533,17 @@ __global__ __launch_bounds__(kQWaves * 64) __attribute__((amdgpu_waves_per_eu((P
   const int grp = g.chunks[m].w, f = grp & 0xFFFF, c = grp >> 16;
   const int off = k - Q * f;
   const int chunk = f + off % c, rg = 8 * (off / c) + xcd;
-  constexpr int NT = 16 * NB;
   // two arrays, not one: the compiler then sees that the direct loads into
   // one buffer cannot alias the reads of the other, and does not wait for
   // them (with all outstanding loads) before the contraction
-  __shared__ __attribute__((aligned(16))) uint8_t lds0[P * NT * kQRowB];
-  __shared__ __attribute__((aligned(16))) uint8_t lds1[P * NT * kQRowB];
-  __shared__ int rows[2 * NT];
-  const int n = g.chunks[chunk].z;
-  if constexpr (NB == 4) {
-    if (n > 48) return qgemm_body<P, 4, DOWN, TL>(g, lds0, lds1, rows, chunk, rg);
-    if (n > 32) return qgemm_body<P, 3, DOWN, TL>(g, lds0, lds1, rows, chunk, rg);
-  }
-  if constexpr (NB >= 2) {
-    if (n > 16) return qgemm_body<P, 2, DOWN, TL>(g, lds0, lds1, rows, chunk, rg);
-  }
-  qgemm_body<P, 1, DOWN, TL>(g, lds0, lds1, rows, chunk, rg);
+  __shared__ __attribute__((aligned(16))) uint8_t lds0[P * 16 * NB * kQRowB];
+  __shared__ __attribute__((aligned(16))) uint8_t lds1[P * 16 * NB * kQRowB];
+  __shared__ int rows[2 * kQMaxTok];
+  const int4 ck = g.chunks[chunk];
+  if (c == 1)
+    qgemm_chunk<P, NB, DOWN, true>(g, lds0, lds1, rows, ck, rg);
+  else
+    qgemm_chunk<P, NB, DOWN, false>(g, lds0, lds1, rows, ck, rg);
 }
 
 hipError_t launch_xplanes(const float* x, int kd, size_t n_rows, int planes, _Float16* xp, float* xs, float* xe,
@@ -491,7 +569,7 @@ int qgemm_chunk_tokens(int planes) { return planes == 3 ? 16 : 64; }
 
 hipError_t launch_qgemm(const QGemmArgs& g, int planes, bool down, int max_chunks, hipStream_t s) {
   const dim3 blk(kQWaves * 64);
-  const int RG = (down ? kHidden : kFfn) / qgemm_rows(qgemm_tiles(planes, down), down);
+  const int RG = (down ? kHidden : kFfn) / qgemm_rows(down);
   const dim3 grid((unsigned)(RG * max_chunks));
   if (planes == 3) {
     if (down)

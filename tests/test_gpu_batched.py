@@ -149,6 +149,42 @@ def test_batched_fp32_grade(fdm, oracle, layer, batch_kernel, T, kind):
         assert m_got <= 4 * m_f32, (t, m_got, m_f32)
 
 
+@pytest.mark.parametrize("n", [1, 5, 6, 10, 11, 16, 17, 22, 27, 32, 33])
+def test_grouped_gemm_chunk_sizes(fdm, oracle, layer, n):
+    """n tokens that all choose the same experts, so every chunk of the
+    grouped GEMMs is n tokens (16 and a remainder above 16): the operand
+    layouts change at 5 / 6 and 10 / 11 tokens.  The tokens are one routing
+    vector plus noise too small to change a choice; every token is held to
+    1e-5 of float64 (the fp32 grade tests pin the paths' own precision)."""
+    import torch
+    L, lay = layer
+    K = 8
+    Wg, bias = to_host(lay.Wg), to_host(lay.bias)
+    rng = np.random.default_rng(n)
+    base = oracle.synth_normal(7168, 0.0, 1.0, 77)
+    X = (base + 1e-3 * rng.standard_normal((n, 7168))).astype(np.float32)
+    out = empty_f32(n * 7168)
+    idx = torch.empty(n * K, dtype=torch.int32, device="cuda")
+    w = empty_f32(n * K)
+    prev = fdm.set_batch_kernel(fdm.BATCH_MFMA)
+    try:
+        say(f"moe_forward_batched L={L} chunk of {n} tokens")
+        fdm.moe_forward_batched(L, to_dev(X.ravel()), None, n, K, out, idx, w)
+    finally:
+        fdm.set_batch_kernel(prev)
+    got, gi, gw = to_host(out).reshape(n, 7168), to_host(idx).reshape(n, K), to_host(w).reshape(n, K)
+    assert len(np.unique(gi)) == K
+    blobs = {e: lay.expert_bytes(e) for e in [-1] + [int(e) for e in gi[0]]}
+    for t in range(n):
+        ri, _ = oracle.route(oracle.router_logits(Wg, X[t]), bias, K=K)
+        assert np.array_equal(gi[t], ri), t
+    for t in sorted({0, n // 3, n // 2, n - 1}):
+        want = np.float64(oracle.expert_ffn(blobs[-1], lay.down_q6, X[t]))
+        for k in range(K):
+            want = want + np.float64(gw[t][k]) * oracle.expert_ffn(blobs[int(gi[t][k])], lay.down_q6, X[t])
+        assert rel_l2(got[t], want) <= 1e-5, t
+
+
 def test_batched_paths_agree(fdm, layer):
     """The two expert paths on the same 96-token step: identical routing,
     outputs within 1e-4 of each other (both carry the activations at fp32
