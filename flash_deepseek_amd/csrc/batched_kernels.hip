@@ -109,8 +109,8 @@ __device__ __forceinline__ int block_scan_excl(int v, int* wsum, int& tot) {
 
 // One workgroup, thread e = expert e: pair counts per expert, segment
 // starts, the ascending list of distinct experts, each pair's position in
-// its expert's segment and, with b.ch > 0, the grouped GEMMs' chunk list
-// (every distinct expert's segment in chunks of b.ch pairs, ascending, then
+// its expert's segment and, with b.ch > 0, the grouped GEMMs' chunk list (with
+// b.ch_down > 0 a second one for the down GEMM; every distinct expert's segment in chunks of b.ch pairs, ascending, then
 // the shared expert's tokens in chunks of b.ch), all by block-wide scans.
 // The order of pairs inside a segment (LDS atomics) does not affect any
 // result: every pair's activations and output come from its own token only.
@@ -152,18 +152,19 @@ __global__ __launch_bounds__(256) void k_dispatch(BatchArgs b) {
     b.seg_start[kExperts] = tot;
     *b.n_distinct = nd;
   }
-  if (b.ch > 0) {
-    const int ch = b.ch;
+  auto chunk_list = [&](int ch, int4* chunks, int* n_chunks) {
     const int nch = (c + ch - 1) / ch;
     int nr;
     const int cpos = block_scan_excl(nch, wsum, nr);
     for (int q = 0; q < nch; ++q)
-      b.chunks[cpos + q] = make_int4(e, st + q * ch, min(ch, c - q * ch), cpos | (nch << 16));
+      chunks[cpos + q] = make_int4(e, st + q * ch, min(ch, c - q * ch), cpos | (nch << 16));
     const int ns = b.shared ? (b.T + ch - 1) / ch : 0;
     for (int q = threadIdx.x; q < ns; q += 256)
-      b.chunks[nr + q] = make_int4(-1, q * ch, min(ch, b.T - q * ch), nr | (ns << 16));
-    if (e == 0) *b.n_chunks = nr + ns;
-  }
+      chunks[nr + q] = make_int4(-1, q * ch, min(ch, b.T - q * ch), nr | (ns << 16));
+    if (e == 0) *n_chunks = nr + ns;
+  };
+  if (b.ch > 0) chunk_list(b.ch, b.chunks, b.n_chunks);
+  if (b.ch_down > 0) chunk_list(b.ch_down, b.chunks_down, b.n_chunks_down);
   __syncthreads();
   auto place = [&](int p, int x) {
     int pos = -1;
@@ -343,19 +344,6 @@ hipError_t launch_combine(const BatchArgs& b, hipStream_t s) {
     hipLaunchKernelGGL(k_bcombine<4>, dim3(kHidden / 1024, b.T), dim3(256), 0, s, b);
   else
     hipLaunchKernelGGL(k_bcombine<1>, dim3(kHidden / 256, b.T), dim3(256), 0, s, b);
-  return hipGetLastError();
-}
-
-hipError_t launch_batched_down(const BatchArgs& b, bool down_q6, hipStream_t s) {
-  const int P = b.T * b.K;
-  const int rows = P + (b.shared ? b.T : 0);
-  const int max_items = (P < kExperts ? P : kExperts) + (b.shared ? (b.T + kBShChunk - 1) / kBShChunk : 0);
-  const int gy = max_items < 16 ? max_items : 16;
-  if (hipError_t e = launch_xdigits(b.act, (size_t)rows * (kFfn / 64), b.act_xd, s)) return e;
-  if (down_q6)
-    hipLaunchKernelGGL(k_bdown<true>, dim3(kBDnTiles, gy), dim3(256), 0, s, b);
-  else
-    hipLaunchKernelGGL(k_bdown<false>, dim3(kBDnTiles, gy), dim3(256), 0, s, b);
   return hipGetLastError();
 }
 

@@ -144,8 +144,8 @@ struct Workspace {
   float* q_xs = nullptr;      // [q_elems / 32] sub-block sums
   float* q_xe = nullptr;      // [q_rows] row scales
   size_t q_rows = 0;
-  int4* q_chunks = nullptr;   // chunk list (kQMaxChunks)
-  int* q_nchunks = nullptr;   // [1]
+  int4* q_chunks = nullptr;   // chunk list (kQMaxChunks), then a second one for the down GEMM
+  int* q_nchunks = nullptr;   // [2]
   // prefill (fdm_moe_prefill)
   int p_tokens = 0;           // tokens the buffer below holds
   float* p_hpost = nullptr;   // [p_tokens][7168] rms_norm output
@@ -315,8 +315,8 @@ int alloc_workspace(Workspace& w) {
   FDM_HIP(hipMalloc(&w.stage_idx, FDM_MAX_K * sizeof(int)));
   FDM_HIP(hipMalloc(&w.stage_w, FDM_MAX_K * sizeof(float)));
   FDM_HIP(hipMalloc(&w.dense_act, kDenseMaxFfn * sizeof(float)));
-  FDM_HIP(hipMalloc(&w.q_chunks, kQMaxChunks * sizeof(int4)));
-  FDM_HIP(hipMalloc(&w.q_nchunks, sizeof(int)));
+  FDM_HIP(hipMalloc(&w.q_chunks, 2 * kQMaxChunks * sizeof(int4)));
+  FDM_HIP(hipMalloc(&w.q_nchunks, 2 * sizeof(int)));
   return FDM_OK;
 }
 
@@ -1507,9 +1507,10 @@ QScratch workspace_q(const Workspace& w) {
 
 // The expert half of one step on the grouped GEMMs, after the dispatch:
 // chunk list, planes of the token rows (unless x_planes_ready: the caller
-// has written them), gate/up + SwiGLU into b.act, then a Q4_K down on the
-// GEMM (planes of b.act first) or a Q6_K down on the dot4 kernels, into
-// b.eo.  x: the fp32 token rows [T][7168].
+// has written them), gate/up + SwiGLU into b.act, the planes of b.act and the
+// down into b.eo.  A Q6_K down takes three planes always, in chunks of their
+// size (one-plane callers have a second chunk list for it in the workspace).
+// x: the fp32 token rows [T][7168].
 int run_qgemm_experts(const Layer* y, const BatchArgs& b0, const float* x, int planes, const QScratch& w,
                       hipStream_t s, bool x_planes_ready = false) {
   BatchArgs b = b0;
@@ -1521,7 +1522,17 @@ int run_qgemm_experts(const Layer* y, const BatchArgs& b0, const float* x, int p
   b.ch = ch;
   b.chunks = w.chunks;
   b.n_chunks = w.n_chunks;
-  FDM_HIP(launch_dispatch(b, s));  // with the chunk list
+  const int planes_down = y->down_q6 ? 3 : planes;
+  const bool own_list = planes_down != planes;
+  int mc_down = mc;
+  if (own_list) {
+    b.ch_down = qgemm_chunk_tokens(planes_down);
+    b.chunks_down = w.chunks + kQMaxChunks;
+    b.n_chunks_down = w.n_chunks + 1;
+    mc_down = max_chunks(T, K, b.ch_down);
+    if (mc_down > kQMaxChunks) return fail(FDM_E_INVAL, "chunk list of %d entries exceeds %d", mc_down, kQMaxChunks);
+  }
+  FDM_HIP(launch_dispatch(b, s));  // with the chunk lists
   if (!x_planes_ready) FDM_HIP(launch_xplanes(x, FDM_HIDDEN, (size_t)T, planes, w.planes, w.xs, w.xe, s));
   QGemmArgs q;
   q.T = T;
@@ -1537,15 +1548,15 @@ int run_qgemm_experts(const Layer* y, const BatchArgs& b0, const float* x, int p
   q.chunks = w.chunks;
   q.n_chunks = w.n_chunks;
   q.out = b.act;
-  FDM_HIP(launch_qgemm(q, planes, false, mc, s));
-  if (y->down_q6) {
-    FDM_HIP(launch_batched_down(b, true, s));
-    return FDM_OK;
-  }
-  FDM_HIP(launch_xplanes(b.act, FDM_MOE_FFN, rows, planes, w.planes, w.xs, w.xe, s));
+  FDM_HIP(launch_qgemm(q, planes, false, false, mc, s));
+  FDM_HIP(launch_xplanes(b.act, FDM_MOE_FFN, rows, planes_down, w.planes, w.xs, w.xe, s));
   q.plane = rows * FDM_MOE_FFN;
   q.out = b.eo;
-  FDM_HIP(launch_qgemm(q, planes, true, mc, s));
+  if (own_list) {
+    q.chunks = b.chunks_down;
+    q.n_chunks = b.n_chunks_down;
+  }
+  FDM_HIP(launch_qgemm(q, planes_down, true, y->down_q6, mc_down, s));
   return FDM_OK;
 }
 }  // namespace

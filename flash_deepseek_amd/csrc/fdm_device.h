@@ -460,10 +460,15 @@ constexpr int kRelGuPieces = 32;
 constexpr int kRelDnPieces = 64;
 
 template <bool DOWN>
-__device__ __forceinline__ const uint8_t* rel_step(const uint8_t* mat, int row, int block) {
+__device__ __forceinline__ size_t rel_step_off(int row, int block) {
   constexpr size_t kStep = 36 * (DOWN ? kRelDnPieces : kRelGuPieces);
-  return mat + (DOWN ? ((size_t)(block >> 2) * (kHidden / 4) + (row >> 2))
-                     : ((size_t)(row >> 1) * (kHidden / 1024) + (block >> 2))) * kStep;
+  return (DOWN ? ((size_t)(block >> 2) * (kHidden / 4) + (row >> 2))
+               : ((size_t)(row >> 1) * (kHidden / 1024) + (block >> 2))) * kStep;
+}
+
+template <bool DOWN>
+__device__ __forceinline__ const uint8_t* rel_step(const uint8_t* mat, int row, int block) {
+  return mat + rel_step_off<DOWN>(row, block);
 }
 
 template <bool DOWN>

@@ -208,10 +208,12 @@ struct BatchArgs {
   int ch = 0;              // tokens per chunk
   int4* chunks = nullptr;  // {expert or -1 (shared), first pair / token, count, first chunk | count << 16}
   int* n_chunks = nullptr;
+  // and a second list, where the down GEMM's chunks are smaller (ch_down > 0)
+  int ch_down = 0;
+  int4* chunks_down = nullptr;
+  int* n_chunks_down = nullptr;
 };
 hipError_t launch_batched_experts(const BatchArgs& b, bool down_q6, hipStream_t s);
-// The grouped down (digits of b.act, then the dot4 down kernel) on its own.
-hipError_t launch_batched_down(const BatchArgs& b, bool down_q6, hipStream_t s);
 // The dispatch and the combine of the batched path on their own (prefill).
 hipError_t launch_dispatch(const BatchArgs& b, hipStream_t s);
 hipError_t launch_combine(const BatchArgs& b, hipStream_t s);
@@ -246,9 +248,9 @@ hipError_t launch_xplanes(const float* x, int kd, size_t n_rows, int planes, _Fl
                           hipStream_t s);
 int qgemm_chunk_tokens(int planes);
 constexpr int kQMaxChunks = 1024;  // >= 256 + 512 * 16 / 16 + 512 / 16
-// Q4_K gate/up + SwiGLU (down = false) or Q4_K down (down = true) over the
-// chunk list; max_chunks bounds the list length.
-hipError_t launch_qgemm(const QGemmArgs& g, int planes, bool down, int max_chunks, hipStream_t s);
+// Q4_K gate/up + SwiGLU (down = false), or the down, Q4_K or (q6, three planes
+// only) Q6_K, over the chunk list; max_chunks bounds the list length.
+hipError_t launch_qgemm(const QGemmArgs& g, int planes, bool down, bool q6, int max_chunks, hipStream_t s);
 
 // dense_kernels.hip: the dense FFN of the first layers (F16 weights)
 constexpr int kDenseMaxFfn = 18432;  // DENSE_INTERMEDIATE (infer.m:59): the down kernel's LDS bound

@@ -1,6 +1,7 @@
 // gemm_kernels.hip -- the grouped expert GEMMs of batched decode and prefill
 // on MFMA: per distinct expert (and the shared one), its tokens' activations
-// against the expert's Q4_K rows, for gate/up (+ SwiGLU) and for a Q4_K down.
+// against the expert's Q4_K rows for gate/up (+ SwiGLU) and its Q4_K or Q6_K
+// rows for the down.
 //
 // Numerics.  Inside one Q4_K block a weight is d*sc*q - dmin*m (quant.c:49-57)
 // with 6-bit sc, m and 4-bit q, so
@@ -16,10 +17,14 @@
 // (Weights carried as 1024 + sc q, with 1024 X cancelled afterwards, would
 // inflate the accumulator several times over the sum it carries and cost
 // the batched path its fp32 grade on SwiGLU activations.)
+// A Q6_K weight is d*sc*(q - 32) with an int8 sc per 16 elements: the integer
+// sc (q - 32), up to 13 significant bits, enters as two halves (build_b6),
+// with no min term.
 // Activations enter as P fp16 planes of x' = x * 2^s (a per-row power of
 // two: the largest |x'| lies in [2^13, 2^14)): P = 3 carries every fp32
-// value exactly (hi + mid + lo, 33 significant bits) -- batched decode, fp32
-// grade; P = 1 carries 11 bits -- prefill, whose bar is 1e-2.  X_sb is the
+// value exactly (hi + mid + lo, 33 significant bits) -- batched decode and
+// every Q6_K down, fp32 grade; P = 1 carries 11 bits -- prefill, whose bar is
+// 1e-2.  X_sb is the
 // fp32 sum of the planes' values.
 //
 // Mapping.  A workgroup of 4 waves owns 64 gate and 64 up rows (wave w:
@@ -54,8 +59,15 @@
 // gate/up of 71 / 132 / 188 experts (16 / 64 / 256 tokens): 328 -> 219, 587 ->
 // 443, 1032 -> 925 us; the down of 16 / 256 tokens 151 -> 122, 517 -> 479 us;
 // one plane, 512 tokens: gate/up 994 -> 906, down 522 -> 499 us.
+// The Q6_K down costs about 200 vector instructions per tile and block (two
+// halves per weight, six bits from two places) and 16 .. 40 MFMAs, and still
+// takes 383 us where the dot4 kernel, which unpacks every weight again for
+// every token, took 922 (132 experts of 64 tokens); 522 against 1906 us for
+// 150 prompt tokens.
 #include "fdm_internal.h"
 #include "planes_device.h"
+
+#include <type_traits>
 
 namespace fdm {
 
@@ -77,10 +89,24 @@ __host__ __device__ constexpr int qgemm_rows(bool down) {  // rows per workgroup
   return (down ? 16 : 8) * kQTiles * kQWaves;
 }
 
-// One lane's share of one block of one weight row (resident expert layout):
-// its group's 32 qs bytes and the 16-byte block header.
+// The matrices a grouped GEMM contracts.
+enum QMat { kGateUp, kDownQ4, kDownQ6 };
+
+// One lane's share of one block of one weight row (resident expert layout).
+// Q4_K: its group's 32 qs bytes (q0, q1) and the 16-byte block header.
+// Q6_K: lane j = 2 h + s holds 16 weights of each quarter k of half h: ql
+// chunk s (q0: quarters 0 and 2), ql chunk 2 + s (q1: quarters 1 and 3) and qh
+// chunk s; hdr = the half's 8 scales and the block's d.
+template <QMat M>
 struct QLane {
   u32x4 q0, q1, hdr;
+};
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+template <>
+struct QLane<kDownQ6> {
+  u32x4 q0, q1, qh;
+  u32x2 sc;
+  uint32_t d;
 };
 
 // fp16 halves of sc * q for the two q held in bits 0-3 (MASK 0x000F000F)
@@ -128,6 +154,77 @@ __device__ __forceinline__ BPair build_b(uint32_t w0, uint32_t w1, f16x2 k_lo, f
   b.lo = __builtin_bit_cast(f16x8, lo);
   b.hi = __builtin_bit_cast(f16x8, hi);
   return b;
+}
+
+// Q6_K: the B operands of MFMA steps m (quarter k = m / 2) and m + 4 (quarter
+// k + 2), m = 2 k + u (k, u = 0, 1): bytes 8 u .. 8 u + 7 of the lane's 16 of
+// each quarter.  A weight's integer is sc (q - 32), up to 4096 in magnitude
+// with 13 significant bits, so two halves carry it exactly: its rounding to
+// 11 bits and what that leaves (-1, 0 or 1).  q is put together in place: four
+// bits of ql at bits 0-3 (4-7 for the high nibbles) and two of qh above
+// them, so (0x6400 | q) - 1056 is q - 32 (and (0x6400 | 16 q) - 1536 is
+// 16 (q - 32)) exactly; then one packed multiply and one packed fma for the
+// rest.  Element order inside each 8 as for Q4_K.
+struct BPair6 {
+  f16x8 lo, lo_r, hi, hi_r;
+};
+
+template <bool HIGH>
+__device__ __forceinline__ void q6_pair(uint32_t l, uint32_t h, f16x2 k, uint32_t& v, uint32_t& r) {
+  uint32_t t;
+  if (HIGH) {
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t) : "v"(l), "s"(0x00F000F0u), "v"(0x64006400u));
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t) : "v"(h), "s"(0x03000300u), "v"(t));
+  } else {
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t) : "v"(l), "s"(0x000F000Fu), "v"(0x64006400u));
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t) : "v"(h), "s"(0x00300030u), "v"(t));
+  }
+  const _Float16 off = HIGH ? (_Float16)-1536.0f : (_Float16)-1056.0f;
+  const f16x2 e = __builtin_bit_cast(f16x2, t) + (f16x2){off, off};
+  const f16x2 a = e * k;
+  v = __builtin_bit_cast(uint32_t, a);
+  r = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(e, k, -a));
+}
+
+// ql dwords w0, w1 and qh dwords h0, h1 of the 8 bytes; SH: the quarter's two
+// qh bits lie at bits 0 (quarters 0 and 2: 0 and 4) or 2 (1 and 3: 2 and 6).
+template <int K>
+__device__ __forceinline__ BPair6 build_b6(uint32_t w0, uint32_t w1, uint32_t h0, uint32_t h1, f16x2 k_lo, f16x2 k_hi) {
+  u32x4 lo, lr, hi, hr;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const uint32_t w = i ? w1 : w0, h = i ? h1 : h0;
+    const uint32_t he = K ? h << 2 : h << 4, ho = K ? h >> 6 : h >> 4, wo = w >> 8;
+    uint32_t v, r;
+    q6_pair<false>(w, he, k_lo, v, r);
+    lo[2 * i] = v, lr[2 * i] = r;
+    q6_pair<false>(wo, ho, k_lo, v, r);
+    lo[2 * i + 1] = v, lr[2 * i + 1] = r;
+    q6_pair<true>(w, he, k_hi, v, r);
+    hi[2 * i] = v, hr[2 * i] = r;
+    q6_pair<true>(wo, ho, k_hi, v, r);
+    hi[2 * i + 1] = v, hr[2 * i + 1] = r;
+  }
+  return BPair6{__builtin_bit_cast(f16x8, lo), __builtin_bit_cast(f16x8, lr), __builtin_bit_cast(f16x8, hi),
+                __builtin_bit_cast(f16x8, hr)};
+}
+
+// Per-block constants of the lane's row: d and, for each quarter k, the
+// lane's 16 weights' scale (its sixteenth for quarters 2 and 3, both in both
+// halves).
+struct QScale6 {
+  float d;
+  f16x2 k[4];
+};
+
+__device__ __forceinline__ QScale6 qscale6(const QLane<kDownQ6>& w, int s) {
+  // the half's scales 2 k + s: bytes s and 2 + s of each dword, signed
+  auto two = [s](uint32_t d) {
+    const uint32_t b = ((d >> (8 * s)) & 0x00FF00FFu) ^ 0x64806480u;  // the halves 1152 + sc
+    return __builtin_bit_cast(f16x2, b) + (f16x2){(_Float16)-1152.0f, (_Float16)-1152.0f};
+  };
+  const f16x2 a = two(w.sc.x), b = two(w.sc.y) * (f16x2){(_Float16)0.0625f, (_Float16)0.0625f};
+  return QScale6{half_to_float(w.d), {(f16x2){a.x, a.x}, (f16x2){a.y, a.y}, (f16x2){b.x, b.x}, (f16x2){b.y, b.y}}};
 }
 
 // Per-block constants of the lane's row and group.
@@ -238,11 +335,12 @@ __global__ __launch_bounds__(256) void k_xplanes(const float* __restrict__ x, si
 // padding would otherwise fill, and are added up once after the last block.
 // NT: the expert has one chunk, its weights are read once and streamed past
 // the L2.
-template <int P, int PK, int NB, bool PACK, bool DOWN, bool NT>
+template <int P, int PK, int NB, bool PACK, QMat M, bool NT>
 __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, uint8_t* lds1, int* rows, const int4 ck,
                                            int rg) {
   static_assert(PACK ? PK == 1 && P == 3 : PK == P, "packed rows carry one plane each");
   constexpr int TL = kQTiles;
+  constexpr bool DOWN = M != kGateUp, Q6 = M == kDownQ6;
   constexpr int KD = DOWN ? kFfn : kHidden;  // contraction length
   constexpr int NBLK = KD / kQK;             // 8 or 28 (even)
   constexpr int NT16 = 16 * NB;              // operand rows per plane slot
@@ -267,31 +365,55 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   const uint8_t* blob = shared ? g.shared : g.experts + (size_t)ck.x * g.expert_size;
   const uint8_t* mat = blob + (DOWN ? 2 * (size_t)kGateBytes : 0);
   constexpr int ROWS = qgemm_rows(DOWN);
-  uint32_t qoff[TL], hoff[TL];
+  uint32_t qoff[TL], hoff[TL], soff[TL];
   int row[TL];
 #pragma unroll
   for (int t = 0; t < TL; ++t) {
     // gate/up: tiles 0 .. TL/2 - 1 gate rows, TL/2 .. TL - 1 the same rows of up
     row[t] = DOWN ? rg * ROWS + 16 * TL * wave + 16 * t + c16 : rg * ROWS + 8 * TL * wave + 16 * (t % (TL / 2)) + c16;
-    const uint32_t base = (uint32_t)(rel_step<DOWN>(nullptr, row[t], 0) - (const uint8_t*)nullptr) +
-                          (!DOWN && t >= TL / 2 ? (uint32_t)kGateBytes : 0u);
-    const int L0 = rel_piece<DOWN>(row[t], 0, 0);
-    qoff[t] = base + 16u * (uint32_t)(L0 + j);
-    hoff[t] = base + 32u * (DOWN ? kRelDnPieces : kRelGuPieces) + 4u * (uint32_t)L0;
+    if constexpr (Q6) {
+      const uint32_t base = (uint32_t)rel6_step_off(row[t], 0), bi = (uint32_t)rel6_block_index(row[t], 0);
+      qoff[t] = base + 16 * (2 * bi + (j >> 1)) + 2048 * (j & 1);
+      soff[t] = base + 16 * bi + 8 * (j >> 1);
+      hoff[t] = base + 2 * bi;
+    } else {
+      const uint32_t base = (uint32_t)rel_step_off<DOWN>(row[t], 0) + (!DOWN && t >= TL / 2 ? (uint32_t)kGateBytes : 0u);
+      const int L0 = rel_piece<DOWN>(row[t], 0, 0);
+      qoff[t] = base + 16u * (uint32_t)(L0 + j);
+      hoff[t] = base + 32u * (DOWN ? kRelDnPieces : kRelGuPieces) + 4u * (uint32_t)L0;
+    }
   }
-  const rsrc_t wr = make_rsrc(mat, (DOWN ? 1 : 2) * (size_t)kGateBytes);
-  auto load_hdr = [&](QLane (&w)[TL], int b) {
-    const uint32_t st = (uint32_t)(rel_step<DOWN>(nullptr, 0, b) - (const uint8_t*)nullptr);
+  const rsrc_t wr = make_rsrc(mat, M == kGateUp ? 2 * (size_t)kGateBytes : Q6 ? kDownQ6KBytes : kDownQ4KBytes);
+  constexpr int NLOADS = (Q6 ? 5 : 3) * TL;  // weight loads per block
+  constexpr int kNt = NT ? kCacheNt : 0;
+  // header of block b, then its quants in the two parts in which a block's
+  // contraction uses them up
+  auto load_hdr = [&](QLane<M> (&w)[TL], int b) {
 #pragma unroll
-    for (int t = 0; t < TL; ++t) w[t].hdr = buf_load16<0>(wr, hoff[t], st + 4 * (uint32_t)rel_piece<DOWN>(0, b, 0));
+    for (int t = 0; t < TL; ++t) {
+      if constexpr (Q6) {
+        const uint32_t st = (uint32_t)rel6_step_off(0, b), bi = (uint32_t)rel6_block_index(0, b);
+        w[t].sc = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_raw_buffer_load_b64(wr, (int)soff[t], (int)(st + kRel6Sc + 16 * bi), 0));
+        w[t].d = __builtin_amdgcn_raw_buffer_load_b16(wr, (int)hoff[t], (int)(st + kRel6D + 2 * bi), 0);
+      } else {
+        w[t].hdr = buf_load16<0>(wr, hoff[t], (uint32_t)rel_step_off<DOWN>(0, b) + 4 * (uint32_t)rel_piece<DOWN>(0, b, 0));
+      }
+    }
   };
-  auto load_q = [&](QLane (&w)[TL], int b, int half) {
-    const uint32_t st = (uint32_t)(rel_step<DOWN>(nullptr, 0, b) - (const uint8_t*)nullptr) +
-                        16 * (uint32_t)(rel_piece<DOWN>(0, b, 0) + half * (DOWN ? kRelDnPieces : kRelGuPieces));
+  auto load_q = [&](QLane<M> (&w)[TL], int b, int part) {
+    const uint32_t st = Q6 ? (uint32_t)rel6_step_off(0, b) + 32 * (uint32_t)rel6_block_index(0, b) + 4096 * part
+                           : (uint32_t)rel_step_off<DOWN>(0, b) +
+                                 16 * (uint32_t)(rel_piece<DOWN>(0, b, 0) + part * (DOWN ? kRelDnPieces : kRelGuPieces));
 #pragma unroll
-    for (int t = 0; t < TL; ++t) (half ? w[t].q1 : w[t].q0) = buf_load16<NT ? kCacheNt : 0>(wr, qoff[t], st);
+    for (int t = 0; t < TL; ++t) {
+      (part ? w[t].q1 : w[t].q0) = buf_load16<kNt>(wr, qoff[t], st);
+      if constexpr (Q6) {
+        if (part) w[t].qh = buf_load16<kNt>(wr, qoff[t], st - 4096 + kRel6Qh);
+      }
+    }
   };
-  QLane wa[TL], wb[TL];
+  QLane<M> wa[TL], wb[TL];
   load_hdr(wa, 0);
   load_q(wa, 0, 0);
   load_q(wa, 0, 1);
@@ -320,7 +442,10 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
     const int p = rho / NT16, r = rho - p * NT16;
     int plane;
     const int t = row_token(r, p, plane);
-    const uint32_t piece = (uint32_t)((lane & 31) ^ (r & 7));
+    uint32_t piece = (uint32_t)((lane & 31) ^ (r & 7));
+    // the Q6_K lane's step m = 2 k + u takes elements 128 h + 32 k + 16 s + 8 u:
+    // kept at piece 8 j + m of the row too
+    if (Q6) piece = 16 * (piece >> 4) + 2 * (piece >> 3 & 1) + 4 * (piece >> 1 & 3) + (piece & 1);
     src[k] = 2u * ((uint32_t)plane * (uint32_t)g.plane + (uint32_t)(rin[t] * KD) + 8u * piece);  // byte offset
   }
   auto dma = [&](int b, int buf) {
@@ -328,12 +453,13 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
 #pragma unroll
     for (int k = 0; k < ROUNDS; ++k) lds_dma16(pr, src[k], (uint32_t)b * (2 * kQK), base + 2 * (wave + kQWaves * k) * kQRowB);
   };
-  const Q4KScaleSel sel = q4k_scale_sel(j);
+  [[maybe_unused]] const Q4KScaleSel sel = q4k_scale_sel(j);
   // corr operand A: plane 0 row c16 of block nb, sub-blocks 2j and 2j+1 of block b
   uint32_t xoff[NBX];
 #pragma unroll
   for (int nb = 0; nb < NBX; ++nb) xoff[nb] = (uint32_t)(rin[min(16 * nb + c16, n - 1)] * (KD / 32) + 2 * j);
   auto load_xs = [&](float2 (&v)[NBX], int b) {
+    if (Q6) return;  // no min term
 #pragma unroll
     for (int nb = 0; nb < NBX; ++nb) {
       v[nb] = *reinterpret_cast<const float2*>(g.xs + 8 * b + xoff[nb]);
@@ -350,14 +476,19 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   // serve every tile, whose B operands are built per step.  With refill, each
   // weight register is loaded with block b + 2 right after its last use: the
   // weight stream runs one to two blocks ahead on two register sets.
-  auto block = [&](int buf, QLane (&w)[TL], const float2 (&xsv)[NBX], bool refill, int b) {
+  auto block = [&](int buf, QLane<M> (&w)[TL], const float2 (&xsv)[NBX], bool refill, int b) {
     const uint8_t* base = buf ? lds1 : lds0;
-    QScale sc[TL];
+    std::conditional_t<Q6, QScale6, QScale> sc[TL];
 #pragma unroll
     for (int t = 0; t < TL; ++t) {
-      sc[t] = qscale(w[t].hdr, sel);
       // every constant is in a register of its own here: the header's are free
-      asm volatile("" : "+v"(sc[t].d), "+v"(sc[t].k_lo), "+v"(sc[t].k_hi), "+v"(sc[t].bc_lo), "+v"(sc[t].bc_hi));
+      if constexpr (Q6) {
+        sc[t] = qscale6(w[t], j & 1);
+        asm volatile("" : "+v"(sc[t].d), "+v"(sc[t].k[0]), "+v"(sc[t].k[1]), "+v"(sc[t].k[2]), "+v"(sc[t].k[3]));
+      } else {
+        sc[t] = qscale(w[t].hdr, sel);
+        asm volatile("" : "+v"(sc[t].d), "+v"(sc[t].k_lo), "+v"(sc[t].k_hi), "+v"(sc[t].bc_lo), "+v"(sc[t].bc_hi));
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
     if (refill) load_hdr(w, b + 2);
@@ -370,23 +501,54 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       const int i0 = 2 * (m & 1);
-      BPair B[TL];
+      auto operand = [&](int p, int nb, int step) {
+        return *reinterpret_cast<const f16x8*>(base + (p * NT16 + 16 * nb + c16) * kQRowB +
+                                               16 * ((8 * j + step) ^ (c16 & 7)));
+      };
+      if constexpr (Q6) {
+        // a tile's four operands are all 16 registers it takes: one tile at a
+        // time, the token operands held
+        f16x8 alo[PK][NB], ahi[PK][NB];
 #pragma unroll
-      for (int t = 0; t < TL; ++t) {
-        const u32x4& q = m < 2 ? w[t].q0 : w[t].q1;
-        B[t] = build_b(q[i0], q[i0 + 1], sc[t].k_lo, sc[t].k_hi);
-      }
+        for (int p = 0; p < PK; ++p)
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
+          for (int nb = 0; nb < NB; ++nb) alo[p][nb] = operand(p, nb, m), ahi[p][nb] = operand(p, nb, m + 4);
 #pragma unroll
-        for (int p = 0; p < PK; ++p) {
-          const uint8_t* r = base + (p * NT16 + 16 * nb + c16) * kQRowB;
-          const f16x8 alo = *reinterpret_cast<const f16x8*>(r + 16 * ((8 * j + m) ^ (c16 & 7)));
-          const f16x8 ahi = *reinterpret_cast<const f16x8*>(r + 16 * ((8 * j + m + 4) ^ (c16 & 7)));
+        for (int t = 0; t < TL; ++t) {
+          const u32x4& q = m < 2 ? w[t].q0 : w[t].q1;
+          const BPair6 B = m < 2 ? build_b6<0>(q[i0], q[i0 + 1], w[t].qh[i0], w[t].qh[i0 + 1], sc[t].k[0], sc[t].k[2])
+                                 : build_b6<1>(q[i0], q[i0 + 1], w[t].qh[i0], w[t].qh[i0 + 1], sc[t].k[1], sc[t].k[3]);
+          // the weights' rest meets the upper 22 bits of the activations
+          // (2^-11 of a weight times 2^-23 of an activation is left out)
 #pragma unroll
-          for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(alo, B[t].lo, C[t][nb]);
+          for (int p = PK - 1; p >= 0; --p) {
 #pragma unroll
-          for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(ahi, B[t].hi, C[t][nb]);
+            for (int nb = 0; nb < NB; ++nb) {
+              if (PK == 1 || p < 2) C[t][nb] = mfma_h(alo[p][nb], B.lo_r, C[t][nb]);
+              C[t][nb] = mfma_h(alo[p][nb], B.lo, C[t][nb]);
+              if (PK == 1 || p < 2) C[t][nb] = mfma_h(ahi[p][nb], B.hi_r, C[t][nb]);
+              C[t][nb] = mfma_h(ahi[p][nb], B.hi, C[t][nb]);
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+        BPair B[TL];
+#pragma unroll
+        for (int t = 0; t < TL; ++t) {
+          const u32x4& q = m < 2 ? w[t].q0 : w[t].q1;
+          B[t] = build_b(q[i0], q[i0 + 1], sc[t].k_lo, sc[t].k_hi);
+        }
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+          for (int p = 0; p < PK; ++p) {
+            const f16x8 alo = operand(p, nb, m), ahi = operand(p, nb, m + 4);
+#pragma unroll
+            for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(alo, B[t].lo, C[t][nb]);
+#pragma unroll
+            for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(ahi, B[t].hi, C[t][nb]);
+          }
         }
       }
       if (refill && (m & 1)) {
@@ -402,9 +564,11 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
         f32x4 a = acc[t][nb];
 #pragma unroll
         for (int i = 0; i < 4; ++i) a[i] = fmaf(sc[t].d, C[t][nb][i], a[i]);
-        if (nb < NBX) {
-          a = mfma_f(xsv[nb].x, sc[t].bc_lo, a);
-          a = mfma_f(xsv[nb].y, sc[t].bc_hi, a);
+        if constexpr (!Q6) {
+          if (nb < NBX) {
+            a = mfma_f(xsv[nb].x, sc[t].bc_lo, a);
+            a = mfma_f(xsv[nb].y, sc[t].bc_hi, a);
+          }
         }
         acc[t][nb] = a;
       }
@@ -417,11 +581,11 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   load_q(wb, 1, 0);
   load_q(wb, 1, 1);
   // Block b from buffer b & 1 while block b + 1 lands in the other one.  The
-  // wait before a block leaves the 3 TL youngest loads in flight (the weights
+  // wait before a block leaves the NLOADS youngest loads in flight (the weights
   // of block b + 1): the loads before them, block b's weights, operands and
   // sub-block sums, have then landed.
   auto pair = [&](int b, bool last) {
-    wait_vm<3 * TL>();
+    wait_vm<NLOADS>();
     __syncthreads();  // block b staged by every wave; buffer 1 read by all (block b - 1)
     dma(b + 1, 1);
     load_xs(xb, b + 1);
@@ -430,7 +594,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
     if (last)
       wait_vm<0>();
     else
-      wait_vm<3 * TL>();
+      wait_vm<NLOADS>();
     __syncthreads();  // block b + 1 staged; buffer 0 read by all (block b)
     if (!last) {
       dma(b + 2, 0);
@@ -439,6 +603,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
     __builtin_amdgcn_sched_barrier(0);
     block(1, wb, xb, !last, b + 1);
   };
+#pragma nounroll
   for (int b = 0; b < NBLK - 2; b += 2) pair(b, false);
   pair(NBLK - 2, true);
   // D of a 16x16 MFMA: lane (c16, j) holds row (column) c16 of the tile and
@@ -502,28 +667,29 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
 // (q = RG / 8), row group 8 ((k - q f) / c) + x of chunk f + (k - q f) % c.
 // An expert's weights are then read from HBM once per row group and served
 // from that XCD's L2 to its other chunks; every XCD does the same work.
-template <int P, int NB, bool DOWN, bool NT>
+template <int P, int NB, QMat M, bool NT>
 __device__ __forceinline__ void qgemm_chunk(const QGemmArgs& g, uint8_t* lds0, uint8_t* lds1, int* rows, const int4 ck,
                                             int rg) {
   const int n = ck.z;
   if constexpr (P == 3) {
-    if (n <= 5) return qgemm_body<3, 1, 1, true, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
-    if (n <= 10) return qgemm_body<3, 1, 2, true, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
-    return qgemm_body<3, 3, 1, false, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
+    if (n <= 5) return qgemm_body<3, 1, 1, true, M, NT>(g, lds0, lds1, rows, ck, rg);
+    if (n <= 10) return qgemm_body<3, 1, 2, true, M, NT>(g, lds0, lds1, rows, ck, rg);
+    return qgemm_body<3, 3, 1, false, M, NT>(g, lds0, lds1, rows, ck, rg);
   } else {
     if constexpr (NB == 4) {
-      if (n > 48) return qgemm_body<P, P, 4, false, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
-      if (n > 32) return qgemm_body<P, P, 3, false, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
+      if (n > 48) return qgemm_body<P, P, 4, false, M, NT>(g, lds0, lds1, rows, ck, rg);
+      if (n > 32) return qgemm_body<P, P, 3, false, M, NT>(g, lds0, lds1, rows, ck, rg);
     }
     if constexpr (NB >= 2) {
-      if (n > 16) return qgemm_body<P, P, 2, false, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
+      if (n > 16) return qgemm_body<P, P, 2, false, M, NT>(g, lds0, lds1, rows, ck, rg);
     }
-    return qgemm_body<P, P, 1, false, DOWN, NT>(g, lds0, lds1, rows, ck, rg);
+    return qgemm_body<P, P, 1, false, M, NT>(g, lds0, lds1, rows, ck, rg);
   }
 }
 
-template <int P, int NB, bool DOWN>
+template <int P, int NB, QMat M>
 __global__ __launch_bounds__(kQWaves * 64) __attribute__((amdgpu_waves_per_eu(qgemm_waves(P)))) void k_qgemm(QGemmArgs g) {
+  constexpr bool DOWN = M != kGateUp;
   constexpr int RG = (DOWN ? kHidden : kFfn) / qgemm_rows(DOWN);
   constexpr int Q = RG / 8;
   static_assert(Q * 8 == RG, "row groups split evenly over the XCDs");
@@ -541,9 +707,9 @@ __global__ __launch_bounds__(kQWaves * 64) __attribute__((amdgpu_waves_per_eu(qg
   __shared__ int rows[2 * kQMaxTok];
   const int4 ck = g.chunks[chunk];
   if (c == 1)
-    qgemm_chunk<P, NB, DOWN, true>(g, lds0, lds1, rows, ck, rg);
+    qgemm_chunk<P, NB, M, true>(g, lds0, lds1, rows, ck, rg);
   else
-    qgemm_chunk<P, NB, DOWN, false>(g, lds0, lds1, rows, ck, rg);
+    qgemm_chunk<P, NB, M, false>(g, lds0, lds1, rows, ck, rg);
 }
 
 hipError_t launch_xplanes(const float* x, int kd, size_t n_rows, int planes, _Float16* xp, float* xs, float* xe,
@@ -567,20 +733,23 @@ hipError_t launch_xplanes(const float* x, int kd, size_t n_rows, int planes, _Fl
 
 int qgemm_chunk_tokens(int planes) { return planes == 3 ? 16 : 64; }
 
-hipError_t launch_qgemm(const QGemmArgs& g, int planes, bool down, int max_chunks, hipStream_t s) {
+hipError_t launch_qgemm(const QGemmArgs& g, int planes, bool down, bool q6, int max_chunks, hipStream_t s) {
   const dim3 blk(kQWaves * 64);
   const int RG = (down ? kHidden : kFfn) / qgemm_rows(down);
   const dim3 grid((unsigned)(RG * max_chunks));
-  if (planes == 3) {
+  if (down && q6) {
+    if (planes != 3) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_qgemm<3, 1, kDownQ6>), grid, blk, 0, s, g);
+  } else if (planes == 3) {
     if (down)
-      hipLaunchKernelGGL((k_qgemm<3, 1, true>), grid, blk, 0, s, g);
+      hipLaunchKernelGGL((k_qgemm<3, 1, kDownQ4>), grid, blk, 0, s, g);
     else
-      hipLaunchKernelGGL((k_qgemm<3, 1, false>), grid, blk, 0, s, g);
+      hipLaunchKernelGGL((k_qgemm<3, 1, kGateUp>), grid, blk, 0, s, g);
   } else {
     if (down)
-      hipLaunchKernelGGL((k_qgemm<1, 4, true>), grid, blk, 0, s, g);
+      hipLaunchKernelGGL((k_qgemm<1, 4, kDownQ4>), grid, blk, 0, s, g);
     else
-      hipLaunchKernelGGL((k_qgemm<1, 4, false>), grid, blk, 0, s, g);
+      hipLaunchKernelGGL((k_qgemm<1, 4, kGateUp>), grid, blk, 0, s, g);
   }
   return hipGetLastError();
 }
