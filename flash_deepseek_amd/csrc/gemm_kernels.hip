@@ -43,7 +43,7 @@
 //
 // What bounds it.  A read of the same weight lines with the same tiles and
 // no math takes 180-205 us for 71 experts' gate and up (5.7-6.6 TB/s); the
-// vector ALU (about 105 instructions per 16-row tile and block, 9 per 8
+// vector ALU (about 95 instructions per 16-row tile and block, 9 per 8
 // weights for the operand) and the matrix cores (16 cycles per 16x16x32, 32
 // per 16x16x4) need about as long and overlap only partly, so the kernel
 // lives on loads in flight and on few instructions:
@@ -54,7 +54,11 @@
 //  - each weight register is refilled with block b + 2 right after its last
 //    use, so the stream runs one to two blocks ahead on two register sets
 //    (234 -> 219 us, 64 tokens 479 -> 443 us);
-//  - buffer loads: no address arithmetic on the vector ALU;
+//  - buffer loads: no address arithmetic on the vector ALU, and a pad row's
+//    planes and sub-block sums lie past the buffer's end, so they cost no
+//    traffic (and the sums no select that waits for the load);
+//  - a block's scales and mins are taken from the header two at a time
+//    (105 -> 95 instructions; 213, 467 and 910 us in the figures below);
 //  - an expert with one chunk is streamed past the L2 (nontemporal).
 // gate/up of 71 / 132 / 188 experts (16 / 64 / 256 tokens): 328 -> 219, 587 ->
 // 443, 1032 -> 925 us; the down of 16 / 256 tokens 151 -> 122, 517 -> 479 us;
@@ -115,17 +119,16 @@ struct QLane<kDownQ6> {
 // gives sc q exactly (q < 16, sc < 64: the exact result is a half, which the
 // single rounding keeps).  For the q in bits 4-7 (MASK 0x00F000F0),
 // 0x6400 | 16 q is the half 1024 + 16 q, and (1024 + 16 q) (sc / 16) - 64 sc
-// is sc q exactly, with no shift to bring the nibble down.  k holds the
-// multiplier in its low half and the addend in its high half; both halves of
-// the fma read them (op_sel).
+// is sc q exactly, with no shift to bring the nibble down.  Both halves of
+// the fma read one half of k and of a (op_sel).
 template <uint32_t MASK>
-__device__ __forceinline__ uint32_t magic2(uint32_t w, f16x2 k) {
+__device__ __forceinline__ uint32_t magic2(uint32_t w, _Float16 k, _Float16 a) {
   // one v_and_or_b32 (mask from an SGPR, 0x64006400 from a VGPR: a VOP3
   // takes no literal and one SGPR), which the compiler otherwise splits
   uint32_t m;
   asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(m) : "v"(w), "s"(MASK), "v"(0x64006400u));
   const f16x2 v = __builtin_bit_cast(f16x2, m);
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, (f16x2){k.x, k.x}, (f16x2){k.y, k.y}));
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, (f16x2){k, k}, (f16x2){a, a}));
 }
 
 // The B operands of MFMA steps m (low nibbles) and m + 4 (high nibbles):
@@ -139,17 +142,17 @@ struct BPair {
   f16x8 lo, hi;
 };
 
-__device__ __forceinline__ BPair build_b(uint32_t w0, uint32_t w1, f16x2 k_lo, f16x2 k_hi) {
+__device__ __forceinline__ BPair build_b(uint32_t w0, uint32_t w1, f16x2 k, f16x2 a) {
   const uint32_t v0 = w0 >> 8, v1 = w1 >> 8;
   u32x4 lo, hi;
-  lo.x = magic2<0x000F000Fu>(w0, k_lo);
-  lo.y = magic2<0x000F000Fu>(v0, k_lo);
-  lo.z = magic2<0x000F000Fu>(w1, k_lo);
-  lo.w = magic2<0x000F000Fu>(v1, k_lo);
-  hi.x = magic2<0x00F000F0u>(w0, k_hi);
-  hi.y = magic2<0x00F000F0u>(v0, k_hi);
-  hi.z = magic2<0x00F000F0u>(w1, k_hi);
-  hi.w = magic2<0x00F000F0u>(v1, k_hi);
+  lo.x = magic2<0x000F000Fu>(w0, k.x, a.x);
+  lo.y = magic2<0x000F000Fu>(v0, k.x, a.x);
+  lo.z = magic2<0x000F000Fu>(w1, k.x, a.x);
+  lo.w = magic2<0x000F000Fu>(v1, k.x, a.x);
+  hi.x = magic2<0x00F000F0u>(w0, k.y, a.y);
+  hi.y = magic2<0x00F000F0u>(v0, k.y, a.y);
+  hi.z = magic2<0x00F000F0u>(w1, k.y, a.y);
+  hi.w = magic2<0x00F000F0u>(v1, k.y, a.y);
   BPair b;
   b.lo = __builtin_bit_cast(f16x8, lo);
   b.hi = __builtin_bit_cast(f16x8, hi);
@@ -227,29 +230,57 @@ __device__ __forceinline__ QScale6 qscale6(const QLane<kDownQ6>& w, int s) {
   return QScale6{half_to_float(w.d), {(f16x2){a.x, a.x}, (f16x2){a.y, a.y}, (f16x2){b.x, b.x}, (f16x2){b.y, b.y}}};
 }
 
-// Per-block constants of the lane's row and group.
+// Per-block constants of the lane's row and group, halves for sub-blocks 2j
+// (low) and 2j + 1 (high).
 struct QScale {
   float d;
-  f16x2 k_lo;          // {sc, -1024 sc} of sub-block 2j
-  f16x2 k_hi;          // {sc / 16, -64 sc} of sub-block 2j+1
-  float bc_lo, bc_hi;  // -dmin m of sub-blocks 2j, 2j+1
+  f16x2 k;             // {sc, sc / 16}
+  f16x2 a;             // {-1024 sc, -64 sc}
+  float bc_lo, bc_hi;  // -dmin m
 };
 
-__device__ __forceinline__ QScale qscale(const u32x4 hdr, const Q4KScaleSel& sel) {
-  int sc0, m0, sc1, m1;
-  q4k_scale_min_pair(hdr.y, hdr.z, hdr.w, sel, sc0, m0, sc1, m1);
+// The scale and min bits of a lane's two sub-blocks, taken from the header's
+// twelve scale bytes two sub-blocks at a time: v_perm_b32 puts the two bytes
+// that hold the low bits (and the two with the top bits of groups 2 and 3)
+// into the two halves of a word.  Selectors and masks are constants of the
+// lane's group g.
+struct QSel {
+  uint32_t lo, top;       // byte selectors
+  uint32_t msk, mshift;   // low bits kept; shift of a min's low bits
+  uint32_t tmsk;          // 0x00300030 where bits 4, 5 come from the top bytes
+};
+__device__ __forceinline__ QSel qsel(int g) {
+  const uint32_t b = 2 * (uint32_t)(g & 1);
+  QSel s;
+  // v_perm_b32 (a, b): selector 0-3 the bytes of b, 4-7 those of a, 12 zero
+  s.top = 0x0C000C00u | (b + 1) << 16 | b;
+  s.lo = g < 2 ? s.top : s.top + 0x00040004u;
+  s.msk = g < 2 ? 0x003F003Fu : 0x000F000Fu;
+  s.mshift = g < 2 ? 0 : 4;
+  s.tmsk = g < 2 ? 0 : 0x00300030u;
+  return s;
+}
+
+__device__ __forceinline__ QScale qscale(const u32x4 hdr, const QSel& sel) {
+  const uint32_t s0 = hdr.y, s1 = hdr.z, s2 = hdr.w;
+  auto six = [&](uint32_t low, uint32_t top) {  // the halves 1024 + v
+    const uint32_t t = __builtin_amdgcn_perm(0u, top, sel.top) >> 2;
+    uint32_t v;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(v) : "v"(low), "v"(sel.msk), "v"(0x64006400u));
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(v) : "v"(t), "v"(sel.tmsk), "v"(v));
+    return __builtin_bit_cast(f16x2, v);
+  };
+  const f16x2 sc = six(__builtin_amdgcn_perm(s2, s0, sel.lo), s0);
+  const f16x2 m = six(__builtin_amdgcn_perm(s2, s1, sel.lo) >> sel.mshift, s1) +
+                  (f16x2){(_Float16)-1024.0f, (_Float16)-1024.0f};
   QScale s;
   s.d = half_to_float(hdr.x);
+  s.k = __builtin_elementwise_fma(sc, (f16x2){(_Float16)1.0f, (_Float16)0.0625f},
+                                  (f16x2){(_Float16)-1024.0f, (_Float16)-64.0f});
+  s.a = s.k * (f16x2){(_Float16)-1024.0f, (_Float16)-1024.0f};
   const float dmin = half_to_float(hdr.x >> 16);
-  // the halves 1024 + sc0 and 1024 + sc1, then {sc0, -1024 sc0} and
-  // {sc1 / 16, -64 sc1}, all exact
-  const f16x2 h = __builtin_bit_cast(f16x2, (uint32_t)sc0 + ((uint32_t)sc1 << 16) + 0x64006400u);
-  const f16x2 k = __builtin_elementwise_fma(h, (f16x2){(_Float16)1.0f, (_Float16)0.0625f},
-                                            (f16x2){(_Float16)-1024.0f, (_Float16)-64.0f});  // {sc0, sc1 / 16}
-  s.k_lo = (f16x2){k.x, k.x * (_Float16)-1024.0f};
-  s.k_hi = (f16x2){k.y, k.y * (_Float16)-1024.0f};
-  s.bc_lo = -(dmin * (float)m0);
-  s.bc_hi = -(dmin * (float)m1);
+  s.bc_lo = fmaf(-dmin, (float)m.x, 0.0f);  // one v_fma_mix_f32 each
+  s.bc_hi = fmaf(-dmin, (float)m.y, 0.0f);
   return s;
 }
 
@@ -418,15 +449,11 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   load_q(wa, 0, 0);
   load_q(wa, 0, 1);
   __syncthreads();  // rin, rout
-  // operand row r of plane slot p -> (plane, token)
+  // operand row r of plane slot p -> (plane, token); token < 0: a pad row
   auto row_token = [&](int r, int p, int& plane) {
-    if (PACK) {
-      r = min(r, 3 * n - 1);
-      plane = (r >= n) + (r >= 2 * n);
-      return r - plane * n;
-    }
-    plane = p;
-    return min(r, n - 1);  // pad rows repeat the last token
+    plane = PACK ? (r >= n) + (r >= 2 * n) : p;
+    const int t = PACK ? r - plane * n : r;
+    return t < n ? t : -1;
   };
   // direct-load sources: round k of wave w fills LDS rows 2 (w + 4 k), +1 of
   // the buffer (row rho = slot * NT16 + r); lane i: row rho0 + i / 32,
@@ -446,25 +473,29 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
     // the Q6_K lane's step m = 2 k + u takes elements 128 h + 32 k + 16 s + 8 u:
     // kept at piece 8 j + m of the row too
     if (Q6) piece = 16 * (piece >> 4) + 2 * (piece >> 3 & 1) + 4 * (piece >> 1 & 3) + (piece & 1);
-    src[k] = 2u * ((uint32_t)plane * (uint32_t)g.plane + (uint32_t)(rin[t] * KD) + 8u * piece);  // byte offset
+    // byte offset; past the buffer's end (no access, zeros) for a pad row
+    src[k] = t < 0 ? 0x80000000u : 2u * ((uint32_t)plane * (uint32_t)g.plane + (uint32_t)(rin[t] * KD) + 8u * piece);
   }
   auto dma = [&](int b, int buf) {
     uint8_t* base = buf ? lds1 : lds0;
 #pragma unroll
     for (int k = 0; k < ROUNDS; ++k) lds_dma16(pr, src[k], (uint32_t)b * (2 * kQK), base + 2 * (wave + kQWaves * k) * kQRowB);
   };
-  [[maybe_unused]] const Q4KScaleSel sel = q4k_scale_sel(j);
-  // corr operand A: plane 0 row c16 of block nb, sub-blocks 2j and 2j+1 of block b
+  [[maybe_unused]] const QSel sel = qsel(j);
+  // corr operand A: plane 0 row c16 of block nb, sub-blocks 2j and 2j+1 of
+  // block b; past the buffer's end (zeros) for a row of another plane or a pad
+  const rsrc_t xr = make_rsrc(g.xs, g.plane / 32 * sizeof(float));
   uint32_t xoff[NBX];
 #pragma unroll
-  for (int nb = 0; nb < NBX; ++nb) xoff[nb] = (uint32_t)(rin[min(16 * nb + c16, n - 1)] * (KD / 32) + 2 * j);
-  auto load_xs = [&](float2 (&v)[NBX], int b) {
+  for (int nb = 0; nb < NBX; ++nb) {
+    const int t = 16 * nb + c16;
+    xoff[nb] = t < n ? 4u * (uint32_t)(rin[t] * (KD / 32) + 2 * j) : 0x80000000u;
+  }
+  auto load_xs = [&](u32x2 (&v)[NBX], int b) {
     if (Q6) return;  // no min term
 #pragma unroll
-    for (int nb = 0; nb < NBX; ++nb) {
-      v[nb] = *reinterpret_cast<const float2*>(g.xs + 8 * b + xoff[nb]);
-      if (PACK && 16 * nb + c16 >= n) v[nb] = float2{0.0f, 0.0f};  // a row of another plane
-    }
+    for (int nb = 0; nb < NBX; ++nb)
+      v[nb] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(xr, (int)xoff[nb], 32 * b, 0));
   };
   f32x4 acc[TL][NB];
 #pragma unroll
@@ -476,7 +507,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   // serve every tile, whose B operands are built per step.  With refill, each
   // weight register is loaded with block b + 2 right after its last use: the
   // weight stream runs one to two blocks ahead on two register sets.
-  auto block = [&](int buf, QLane<M> (&w)[TL], const float2 (&xsv)[NBX], bool refill, int b) {
+  auto block = [&](int buf, QLane<M> (&w)[TL], const u32x2 (&xsv)[NBX], bool refill, int b) {
     const uint8_t* base = buf ? lds1 : lds0;
     std::conditional_t<Q6, QScale6, QScale> sc[TL];
 #pragma unroll
@@ -487,7 +518,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
         asm volatile("" : "+v"(sc[t].d), "+v"(sc[t].k[0]), "+v"(sc[t].k[1]), "+v"(sc[t].k[2]), "+v"(sc[t].k[3]));
       } else {
         sc[t] = qscale(w[t].hdr, sel);
-        asm volatile("" : "+v"(sc[t].d), "+v"(sc[t].k_lo), "+v"(sc[t].k_hi), "+v"(sc[t].bc_lo), "+v"(sc[t].bc_hi));
+        asm volatile("" : "+v"(sc[t].d), "+v"(sc[t].k), "+v"(sc[t].a), "+v"(sc[t].bc_lo), "+v"(sc[t].bc_hi));
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -537,7 +568,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
 #pragma unroll
         for (int t = 0; t < TL; ++t) {
           const u32x4& q = m < 2 ? w[t].q0 : w[t].q1;
-          B[t] = build_b(q[i0], q[i0 + 1], sc[t].k_lo, sc[t].k_hi);
+          B[t] = build_b(q[i0], q[i0 + 1], sc[t].k, sc[t].a);
         }
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
@@ -566,8 +597,8 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
         for (int i = 0; i < 4; ++i) a[i] = fmaf(sc[t].d, C[t][nb][i], a[i]);
         if constexpr (!Q6) {
           if (nb < NBX) {
-            a = mfma_f(xsv[nb].x, sc[t].bc_lo, a);
-            a = mfma_f(xsv[nb].y, sc[t].bc_hi, a);
+            a = mfma_f(__uint_as_float(xsv[nb].x), sc[t].bc_lo, a);
+            a = mfma_f(__uint_as_float(xsv[nb].y), sc[t].bc_hi, a);
           }
         }
         acc[t][nb] = a;
@@ -575,7 +606,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   };
 
   dma(0, 0);
-  float2 xa[NBX], xb[NBX];
+  u32x2 xa[NBX], xb[NBX];
   load_xs(xa, 0);
   load_hdr(wb, 1);
   load_q(wb, 1, 0);
