@@ -689,15 +689,21 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
 // 3 n packed rows up to 10 tokens; from 11 on the packed rows fill three
 // blocks too, and the planes of a token accumulate in registers), so its
 // weight operands are built once for up to 64 tokens and no MFMA runs on an
-// empty block.  One-dimensional grid, mapped so that all the
-// chunks of one expert that share a row group run on the same XCD, back to
-// back: workgroups are handed to the eight XCDs in turn (id % 8), so
-// id -> (xcd = id % 8, k = id / 8); XCD x owns row groups x, x + 8, ...
-// (RG / 8 of them) of every chunk, and its k-th item is, within the item
-// range q f .. q (f + c) - 1 of the expert whose chunks are f .. f + c - 1
-// (q = RG / 8), row group 8 ((k - q f) / c) + x of chunk f + (k - q f) % c.
-// An expert's weights are then read from HBM once per row group and served
-// from that XCD's L2 to its other chunks; every XCD does the same work.
+// empty block.
+// One-dimensional grid: workgroups are handed to the eight XCDs in turn
+// (id % 8), so id -> (xcd = id % 8, k = id / 8).  The items of an expert whose
+// chunks are f .. f + c - 1 are ordered row group by row group, its chunks
+// back to back, so its weights are read from HBM once per row group and
+// served from that XCD's L2 to its other chunks.
+// Three planes of Q4_K rows: the items of all experts in one row, cut into eight equal
+// ranges, one per XCD.  An expert's token planes (up to 690 KB of 16 tokens)
+// are then read by one XCD or two instead of all eight (gate/up of 256 tokens
+// fetches 3.85 GB instead of 4.44; 16 / 64 / 256 tokens 221 -> 210, 474 -> 457,
+// 873 -> 853 us; the down 121 -> 110 and 458 -> 438 us for 16 and 256).
+// One plane, and the Q6_K down: XCD x has row groups x, x + 8, .. of every
+// chunk.  Chunks of up to 64 tokens differ fourfold in cost, and equal ranges
+// of them left XCDs idle at the end (512 tokens: 829 -> 860 us); the Q6_K down
+// reads more weights per token plane (384 -> 387 us, 1080 -> 1090 at 512).
 template <int P, int NB, QMat M, bool NT>
 __device__ __forceinline__ void qgemm_chunk(const QGemmArgs& g, uint8_t* lds0, uint8_t* lds1, int* rows, const int4 ck,
                                             int rg) {
@@ -724,12 +730,21 @@ __global__ __launch_bounds__(kQWaves * 64) __attribute__((amdgpu_waves_per_eu(qg
   constexpr int RG = (DOWN ? kHidden : kFfn) / qgemm_rows(DOWN);
   constexpr int Q = RG / 8;
   static_assert(Q * 8 == RG, "row groups split evenly over the XCDs");
-  const int id = blockIdx.x, xcd = id & 7, k = id >> 3;
-  const int m = k / Q;  // a chunk of the item's expert
-  if (m >= *g.n_chunks) return;
-  const int grp = g.chunks[m].w, f = grp & 0xFFFF, c = grp >> 16;
-  const int off = k - Q * f;
-  const int chunk = f + off % c, rg = 8 * (off / c) + xcd;
+  const int id = blockIdx.x, xcd = id & 7, k = id >> 3, n_chunks = *g.n_chunks;
+  int chunk, rg, c;
+  if constexpr (P == 3 && M != kDownQ6) {
+    const int items = n_chunks * RG, per = (items + 7) >> 3, item = xcd * per + k;
+    if (k >= per || item >= items) return;
+    const int grp = g.chunks[item / RG].w, f = grp & 0xFFFF, off = item - RG * f;
+    c = grp >> 16;
+    chunk = f + off % c, rg = off / c;
+  } else {
+    const int m = k / Q;  // a chunk of the item's expert
+    if (m >= n_chunks) return;
+    const int grp = g.chunks[m].w, f = grp & 0xFFFF, off = k - Q * f;
+    c = grp >> 16;
+    chunk = f + off % c, rg = 8 * (off / c) + xcd;
+  }
   // two arrays, not one: the compiler then sees that the direct loads into
   // one buffer cannot alias the reads of the other, and does not wait for
   // them (with all outstanding loads) before the contraction
