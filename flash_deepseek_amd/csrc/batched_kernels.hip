@@ -202,9 +202,8 @@ __global__ __launch_bounds__(256) void k_bgateup(BatchArgs b) {
     const ItemRows r = item_rows(b, d, D, &e);
     const uint8_t* blob = r.shared ? b.shared : b.experts + (size_t)e * b.expert_size;
     Q4KGroupLoad ld[7];
-    const uint8_t* mat = blob + (q >= 2 ? kGateBytes : 0);
 #pragma unroll
-    for (int i = 0; i < 7; ++i) ld[i] = rel_load_group<false>(mat, row, 4 * i + (l16 >> 2), g);
+    for (int i = 0; i < 7; ++i) ld[i] = rel_load_group<false>(blob, row, 4 * i + (l16 >> 2), g, q >= 2);
     auto tok_of = [&](int i) { return r.shared ? r.first + i : b.pair_tok[r.first + i]; };
     Records<kHidden / 64> rec;
     rec.load(b.xd + (size_t)tok_of(0) * (kHidden / 64));

@@ -436,56 +436,58 @@ __device__ __forceinline__ void q4k_group_dot_rows(const Q4KGroupLoad (&ld)[R], 
 
 
 // ---- the resident expert layout (REL) ---------------------------------------------------
-// Experts of a resident layer are stored with each Q4_K matrix permuted so
-// that every load instruction of the dot4 kernels reads whole contiguous
-// lines: in the packed layout a half-wave's 16-byte loads hit every other
-// 16 bytes of several rows, so lines are fetched twice and the streaming
-// ("nt") cache policy cannot be used; in REL a half-wave (gate/up) or a
-// wave (down) reads one contiguous run, and nontemporal loads stream ~20%
-// faster.  The values are untouched: REL is a permutation of the packed
+// Experts of a resident layer are stored with their Q4_K matrices permuted so
+// that every load instruction reads whole contiguous lines: in the packed
+// layout a wave's 16-byte loads hit every other 16 bytes of several rows, so
+// lines are fetched twice and the streaming ("nt") cache policy cannot be
+// used; in REL a wave reads one contiguous run, and nontemporal loads stream
+// ~20% faster.  The values are untouched: REL is a permutation of the packed
 // blob's bytes, made once when a layer becomes resident.
-//  gate / up [2048 x 7168] (28 blocks per row): step (row / 2, block / 4),
-//    N = 32 pieces, at ((row / 2) * 7 + block / 4) * 1152.
-//  down Q4_K [7168 x 2048] (8 blocks per row): step (block / 4, row / 4),
-//    N = 64 pieces, at ((block / 4) * 1792 + row / 4) * 2304.
-//  Inside a step (36 N bytes): the first 16 qs bytes of group g of each
-//  piece at 16 L, the last 16 at 16 N + 16 L, header dword g at 32 N + 4 L,
-//  where L = (block % 4) * 4 R + (row % R) * 4 + g (R = 2 rows for gate /
-//  up, 4 for down): one block of a step's rows fills whole 128-byte lines of
-//  q0 and of q1, so a kernel that walks the blocks one at a time (the
-//  grouped GEMMs) reads every line at once instead of half of it now and
-//  the other half a block later, after the L2 may have dropped it.  A Q6_K
+//  A step holds four rows x four blocks, 64 blocks x groups, in 2304 B:
+//  gate and up [2048 x 7168] together (28 blocks per row): step (row / 2,
+//    block / 4) at ((row / 2) * 7 + block / 4) * 2304 of the blob, its rows
+//    ri = 0, 1 the gate's and 2, 3 the up's two;
+//  down Q4_K [7168 x 2048] (8 blocks per row): step (block / 4, row / 4) at
+//    ((block / 4) * 1792 + row / 4) * 2304 of the matrix, ri = row % 4.
+//  Inside a step: the first 16 qs bytes of group g of (row ri, block) at
+//  16 L, the last 16 at 1024 + 16 L, L = (block % 4) * 16 + 4 g + ri; the
+//  16-byte header at 2048 + 16 ((block % 4) * 4 + ri).  One block of a step's
+//  rows fills whole 128-byte lines of q0 and of q1, so a kernel that walks
+//  the blocks one at a time (the grouped GEMMs) reads every line at once
+//  instead of half of it now and the other half a block later, after the L2
+//  may have dropped it.  The rows are the fastest index because four
+//  consecutive lanes of an MFMA operand hold one group of four rows: they
+//  read one 64-byte run, where with the groups fastest each of them hit
+//  another line and a 1 KB load took 30 L1 cycles instead of 17.  A Q6_K
 //  down matrix has a layout of its own (below).
-constexpr int kRelGuPieces = 32;
-constexpr int kRelDnPieces = 64;
+constexpr int kRelStep = 2304, kRelQ1 = 1024, kRelHdr = 2048;
 
 template <bool DOWN>
 __device__ __forceinline__ size_t rel_step_off(int row, int block) {
-  constexpr size_t kStep = 36 * (DOWN ? kRelDnPieces : kRelGuPieces);
   return (DOWN ? ((size_t)(block >> 2) * (kHidden / 4) + (row >> 2))
-               : ((size_t)(row >> 1) * (kHidden / 1024) + (block >> 2))) * kStep;
+               : ((size_t)(row >> 1) * (kHidden / 1024) + (block >> 2))) * kRelStep;
 }
 
+// A row's place in its steps.
 template <bool DOWN>
-__device__ __forceinline__ const uint8_t* rel_step(const uint8_t* mat, int row, int block) {
-  return mat + rel_step_off<DOWN>(row, block);
+__device__ __forceinline__ int rel_row(int row, bool up) {
+  return DOWN ? row & 3 : (row & 1) + (up ? 2 : 0);
 }
 
-template <bool DOWN>
-__device__ __forceinline__ int rel_piece(int row, int block, int g) {
-  return DOWN ? (block & 3) * 16 + (row & 3) * 4 + g : (block & 3) * 8 + (row & 1) * 4 + g;
-}
+__device__ __forceinline__ int rel_piece(int ri, int block, int g) { return (block & 3) * 16 + 4 * g + ri; }
 
-// Group g of block `block` of row `row` of a REL matrix, by nontemporal loads.
+// Group g of block `block` of row `row`, by nontemporal loads.  base: the blob
+// for a gate (up = false) or up row, the down matrix for a down row.
 template <bool DOWN>
-__device__ __forceinline__ Q4KGroupLoad rel_load_group(const uint8_t* mat, int row, int block, int g) {
-  constexpr int N = DOWN ? kRelDnPieces : kRelGuPieces;
-  const uint8_t* s = rel_step<DOWN>(mat, row, block);
-  const int L = rel_piece<DOWN>(row, block, g);
+__device__ __forceinline__ Q4KGroupLoad rel_load_group(const uint8_t* base, int row, int block, int g,
+                                                       bool up = false) {
+  const uint8_t* s = base + rel_step_off<DOWN>(row, block);
+  const int ri = rel_row<DOWN>(row, up), L = rel_piece(ri, block, g);
   Q4KGroupLoad r;
-  r.hdr_part = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(s + 32 * N + 4 * L));
+  r.hdr_part = __builtin_nontemporal_load(
+      reinterpret_cast<const uint32_t*>(s + kRelHdr + 16 * ((block & 3) * 4 + ri) + 4 * g));
   r.q0 = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(s + 16 * L));
-  r.q1 = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(s + 16 * N + 16 * L));
+  r.q1 = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(s + kRelQ1 + 16 * L));
   return r;
 }
 

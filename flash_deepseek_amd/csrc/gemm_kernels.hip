@@ -28,13 +28,14 @@
 // fp32 sum of the planes' values.
 //
 // Mapping.  A workgroup of 4 waves owns 64 gate and 64 up rows (wave w:
-// rows 16 w .. 16 w + 15 of both, so SwiGLU is applied in registers) or 128
-// down rows (wave w: two tiles of 16) for one chunk of tokens of one expert.
+// rows 16 w .. 16 w + 15 of both, two of gate and the same two of up by turns
+// in its two 16-column tiles, as the resident layout holds them) or 128 down
+// rows (wave w: two tiles of 16) for one chunk of tokens of one expert.
 // Weight rows are the MFMA columns (B operand): lane (c, j)
 // holds row c and group j (qs bytes 32 j .. 32 j + 31, sub-blocks 2j, 2j+1)
 // of every block, read as two whole 16-byte pieces of the resident expert
-// layout, so the four lanes of a row read one 64-byte line per load and
-// each lane needs only its own group's two scales and mins.  MFMA step m
+// layout: four consecutive lanes, four rows' group j, read one 64-byte run,
+// and each lane needs only its own group's two scales and mins.  MFMA step m
 // (0..7) of a block takes from lane j the 8 elements 64 j + 8 m .. + 7 (low
 // nibbles for m < 4, high nibbles for m >= 4); the token operand (A, from
 // LDS) reads the same elements.  Per block the chunk's token planes are
@@ -59,6 +60,8 @@
 //    traffic (and the sums no select that waits for the load);
 //  - a block's scales and mins are taken from the header two at a time
 //    (105 -> 95 instructions; 213, 467 and 910 us in the figures below);
+//  - the resident layout's row-fastest pieces halve the L1 cycles of a weight
+//    load (16 / 64 / 256 tokens 210 -> 199, 468 -> 444, 883 -> 855 us);
 //  - an expert with one chunk is streamed past the L2 (nontemporal).
 // gate/up of 71 / 132 / 188 experts (16 / 64 / 256 tokens): 328 -> 219, 587 ->
 // 443, 1032 -> 925 us; the down of 16 / 256 tokens 151 -> 122, 517 -> 479 us;
@@ -83,8 +86,8 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 constexpr int kQWaves = 4;            // waves per workgroup
 constexpr int kQRowB = kQK * 2;       // LDS token row: one block of fp16 (512 B)
 constexpr int kQMaxTok = 64;          // tokens of the largest chunk
-// Weight tiles of 16 rows per wave: one of gate and one of up (SwiGLU pairs
-// them), or two of down; every token operand read from LDS serves both.
+// Weight tiles of 16 columns per wave: two of gate/up (8 rows of each, gate
+// and up by turns of two), or two of down; every token operand read from LDS serves both.
 constexpr int kQTiles = 2;
 // Waves per SIMD: 3 for three planes (168 VGPRs), 2 for one plane, whose
 // 64-token chunks hold four operand blocks of accumulators.
@@ -400,18 +403,19 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   int row[TL];
 #pragma unroll
   for (int t = 0; t < TL; ++t) {
-    // gate/up: tiles 0 .. TL/2 - 1 gate rows, TL/2 .. TL - 1 the same rows of up
-    row[t] = DOWN ? rg * ROWS + 16 * TL * wave + 16 * t + c16 : rg * ROWS + 8 * TL * wave + 16 * (t % (TL / 2)) + c16;
+    // gate/up: column c16 of tile t is row 2 (4 t + c16 / 4) + c16 % 2 of the
+    // wave's 16, of gate for c16 % 4 < 2, else of up
+    row[t] = DOWN ? rg * ROWS + 16 * TL * wave + 16 * t + c16
+                  : rg * ROWS + 8 * TL * wave + 8 * t + 2 * (c16 >> 2) + (c16 & 1);
     if constexpr (Q6) {
       const uint32_t base = (uint32_t)rel6_step_off(row[t], 0), bi = (uint32_t)rel6_block_index(row[t], 0);
       qoff[t] = base + 16 * (2 * bi + (j >> 1)) + 2048 * (j & 1);
       soff[t] = base + 16 * bi + 8 * (j >> 1);
       hoff[t] = base + 2 * bi;
     } else {
-      const uint32_t base = (uint32_t)rel_step_off<DOWN>(row[t], 0) + (!DOWN && t >= TL / 2 ? (uint32_t)kGateBytes : 0u);
-      const int L0 = rel_piece<DOWN>(row[t], 0, 0);
-      qoff[t] = base + 16u * (uint32_t)(L0 + j);
-      hoff[t] = base + 32u * (DOWN ? kRelDnPieces : kRelGuPieces) + 4u * (uint32_t)L0;
+      const uint32_t base = (uint32_t)rel_step_off<DOWN>(row[t], 0), ri = c16 & 3;
+      qoff[t] = base + 16 * (uint32_t)rel_piece((int)ri, 0, j);
+      hoff[t] = base + kRelHdr + 16 * ri;
     }
   }
   const rsrc_t wr = make_rsrc(mat, M == kGateUp ? 2 * (size_t)kGateBytes : Q6 ? kDownQ6KBytes : kDownQ4KBytes);
@@ -428,14 +432,13 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
             u32x2, __builtin_amdgcn_raw_buffer_load_b64(wr, (int)soff[t], (int)(st + kRel6Sc + 16 * bi), 0));
         w[t].d = __builtin_amdgcn_raw_buffer_load_b16(wr, (int)hoff[t], (int)(st + kRel6D + 2 * bi), 0);
       } else {
-        w[t].hdr = buf_load16<0>(wr, hoff[t], (uint32_t)rel_step_off<DOWN>(0, b) + 4 * (uint32_t)rel_piece<DOWN>(0, b, 0));
+        w[t].hdr = buf_load16<0>(wr, hoff[t], (uint32_t)rel_step_off<DOWN>(0, b) + 64 * (uint32_t)(b & 3));
       }
     }
   };
   auto load_q = [&](QLane<M> (&w)[TL], int b, int part) {
     const uint32_t st = Q6 ? (uint32_t)rel6_step_off(0, b) + 32 * (uint32_t)rel6_block_index(0, b) + 4096 * part
-                           : (uint32_t)rel_step_off<DOWN>(0, b) +
-                                 16 * (uint32_t)(rel_piece<DOWN>(0, b, 0) + part * (DOWN ? kRelDnPieces : kRelGuPieces));
+                           : (uint32_t)rel_step_off<DOWN>(0, b) + 256 * (uint32_t)(b & 3) + kRelQ1 * part;
 #pragma unroll
     for (int t = 0; t < TL; ++t) {
       (part ? w[t].q1 : w[t].q0) = buf_load16<kNt>(wr, qoff[t], st);
@@ -646,37 +649,45 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
     else
       g.out[(size_t)rout[t] * kFfn + row[tile]] = silu_mul(gate * e, up * e);
   };
-  constexpr int OT = DOWN ? TL : TL / 2;  // output tiles
+  // gate/up: the up value of a gate lane's row lies two lanes on
+  const bool writer = DOWN || (c16 & 2) == 0;
+  auto up_of = [](float v) {
+    return DOWN ? 0.0f : __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xEE, 0xF, 0xF, false));
+  };
   if constexpr (!PACK) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int t = 16 * nb + 4 * j + i;
-        if (t >= n) continue;
+        float up[TL];
 #pragma unroll
-        for (int tt = 0; tt < OT; ++tt) put(t, tt, acc[tt][nb][i], DOWN ? 0.0f : acc[DOWN ? tt : tt + TL / 2][nb][i]);
+        for (int tt = 0; tt < TL; ++tt) up[tt] = up_of(acc[tt][nb][i]);
+        if (t >= n || !writer) continue;
+#pragma unroll
+        for (int tt = 0; tt < TL; ++tt) put(t, tt, acc[tt][nb][i], up[tt]);
       }
     }
   } else {
     // the three planes of a token lie in other lanes' rows: through a
     // wave-private piece of buffer 0 (no longer read or written: the last
     // block is in buffer 1), tile by tile
-    float* red = reinterpret_cast<float*>(lds0) + wave * (DOWN ? 1 : 2) * NT16 * 16;
+    float* red = reinterpret_cast<float*>(lds0) + wave * NT16 * 16;
 #pragma unroll
-    for (int tt = 0; tt < OT; ++tt) {
+    for (int tt = 0; tt < TL; ++tt) {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int r = 16 * nb + 4 * j + i;
           red[r * 16 + c16] = acc[tt][nb][i];
-          if (!DOWN) red[(NT16 + r) * 16 + c16] = acc[DOWN ? tt : tt + TL / 2][nb][i];
         }
       auto sum = [&](const float* p) { return (p[2 * n * 16] + p[n * 16]) + p[0]; };
-      for (int t = j; t < n; t += 4) {
-        const float* p = red + t * 16 + c16;
-        put(t, tt, sum(p), DOWN ? 0.0f : sum(p + NT16 * 16));
+      if (writer) {
+        for (int t = j; t < n; t += 4) {
+          const float* p = red + t * 16 + c16;
+          put(t, tt, sum(p), DOWN ? 0.0f : sum(p + 2));
+        }
       }
       __builtin_amdgcn_wave_barrier();  // the next tile's values overwrite these
     }

@@ -503,10 +503,9 @@ __device__ __forceinline__ void gateup_run(const LayerArgs& a, int slot, int til
   for (int t = 0; t < kGuPer; ++t) {
     const int row = (tile0 + t) * kGuTileRows + 2 * wave + (q & 1);
     Q4KGroupLoad ld[7];
-    // resident expert layout: each half-wave load reads one 512-byte run
-    const uint8_t* mat = src + (q >= 2 ? kGateBytes : 0);
+    // resident expert layout: each wave load reads one 1 KB run
 #pragma unroll
-    for (int i = 0; i < 7; ++i) ld[i] = rel_load_group<false>(mat, row, 4 * i + (l16 >> 2), g);
+    for (int i = 0; i < 7; ++i) ld[i] = rel_load_group<false>(src, row, 4 * i + (l16 >> 2), g, q >= 2);
     if (t == 0) {
       if (!ROUTED) {
         wait_route_xd(a, slot, false, true, sm);

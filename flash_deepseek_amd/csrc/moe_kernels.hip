@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256) void k_gateup(SlotTable t, const XGroup* __res
     const uint8_t* rowp = mat + (size_t)row * kQ4KRowHidden;
 #pragma unroll
     for (int i = 0; i < 7; ++i)
-      ld[i] = t.rel ? rel_load_group<false>(mat, row, 4 * i + (l16 >> 2), g)
+      ld[i] = t.rel ? rel_load_group<false>(blob, row, 4 * i + (l16 >> 2), g, q >= 2)
                     : q4k_load_group(rowp + (4 * i + (l16 >> 2)) * kQ4KBlock, g);
   }
   st.store(xs, kHidden / 64);

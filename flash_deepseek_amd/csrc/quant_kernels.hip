@@ -81,7 +81,7 @@ __global__ __launch_bounds__(256) void k_dequant_q6k(const uint8_t* __restrict__
 // ---- packed blobs -> the resident expert layout (REL) ----------------------------------
 // One thread per Q4_K block of a blob's gate, up or Q4_K down matrix: the
 // block's header dwords and its 8 half-groups go to their REL pieces (see
-// rel_step / rel_piece).  Blob b of n: src + b * src_stride ->
+// rel_step_off / rel_piece).  Blob b of n: src + b * src_stride ->
 // dst + b * expert_size.  A Q6_K down matrix goes through k_rel_pack_q6.
 __global__ __launch_bounds__(256) void k_rel_pack(const uint8_t* __restrict__ src, size_t src_stride,
                                                   uint8_t* __restrict__ dst, size_t expert_size,
@@ -98,35 +98,34 @@ __global__ __launch_bounds__(256) void k_rel_pack(const uint8_t* __restrict__ sr
     uint8_t* db = dst + (size_t)b * expert_size;
     const u32x4* blk;
     uint8_t* step;
-    int L, N;
+    int ri, block;
     if (k < 2 * kGuBlocks) {
       const int m = k / kGuBlocks;  // 0 gate, 1 up
       k %= kGuBlocks;
-      const int row = k / (kHidden / kQK), block = k % (kHidden / kQK);
-      const size_t mo = (size_t)m * kGateBytes;
-      blk = reinterpret_cast<const u32x4*>(sb + mo + (size_t)row * kQ4KRowHidden + block * kQ4KBlock);
-      step = const_cast<uint8_t*>(rel_step<false>(db + mo, row, block));
-      L = rel_piece<false>(row, block, 0);
-      N = kRelGuPieces;
+      const int row = k / (kHidden / kQK);
+      block = k % (kHidden / kQK);
+      blk = reinterpret_cast<const u32x4*>(sb + (size_t)m * kGateBytes + (size_t)row * kQ4KRowHidden + block * kQ4KBlock);
+      step = db + rel_step_off<false>(row, block);
+      ri = rel_row<false>(row, m == 1);
     } else {
       k -= 2 * kGuBlocks;
-      const int row = k / (kFfn / kQK), block = k % (kFfn / kQK);
+      const int row = k / (kFfn / kQK);
+      block = k % (kFfn / kQK);
       const size_t mo = 2 * (size_t)kGateBytes;
       blk = reinterpret_cast<const u32x4*>(sb + mo + (size_t)row * kQ4KRowFfn + block * kQ4KBlock);
-      step = const_cast<uint8_t*>(rel_step<true>(db + mo, row, block));
-      L = rel_piece<true>(row, block, 0);
-      N = kRelDnPieces;
+      step = db + mo + rel_step_off<true>(row, block);
+      ri = rel_row<true>(row, false);
     }
     u32x4 v[9];
 #pragma unroll
     for (int j = 0; j < 9; ++j) v[j] = blk[j];
-    // header dwords g = 0..3 (pieces L + g are consecutive)
-    *reinterpret_cast<u32x4*>(step + 32 * N + 4 * L) = v[0];
+    *reinterpret_cast<u32x4*>(step + kRelHdr + 16 * ((block & 3) * 4 + ri)) = v[0];
     // qs of group g: bytes 32 g .. 32 g + 31 of the block's qs = v[1 + 2 g], v[2 + 2 g]
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      *reinterpret_cast<u32x4*>(step + 16 * (L + g)) = v[1 + 2 * g];
-      *reinterpret_cast<u32x4*>(step + 16 * N + 16 * (L + g)) = v[2 + 2 * g];
+      uint8_t* p = step + 16 * rel_piece(ri, block, g);
+      *reinterpret_cast<u32x4*>(p) = v[1 + 2 * g];
+      *reinterpret_cast<u32x4*>(p + kRelQ1) = v[2 + 2 * g];
     }
   }
 }
