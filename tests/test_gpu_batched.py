@@ -185,6 +185,29 @@ def test_grouped_gemm_chunk_sizes(fdm, oracle, layer, n):
         assert rel_l2(got[t], want) <= 1e-5, t
 
 
+@pytest.mark.parametrize("T,K", [(40, 8), (256, 8), (512, 16)])
+def test_grouped_gemm_repeats_bit_exact(fdm, layer, T, K):
+    """The same step gives the same bits every time: experts with more than
+    one chunk get their tokens in the same order.  (512, 16) has more pairs
+    than the dispatch holds in registers."""
+    import torch
+    from flash_deepseek_amd.synthetic import make_tokens
+    L, _ = layer
+    X = make_tokens(T, 6000 + T)
+    prev = fdm.set_batch_kernel(fdm.BATCH_MFMA)
+    try:
+        outs = []
+        for rep in range(4):
+            out = empty_f32(T * 7168)
+            say(f"moe_forward_batched L={L} T={T} K={K} pass {rep}")
+            fdm.moe_forward_batched(L, X, None, T, K, out)
+            outs.append(out)
+    finally:
+        fdm.set_batch_kernel(prev)
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+
+
 def test_batched_paths_agree(fdm, layer):
     """The two expert paths on the same 96-token step: identical routing,
     outputs within 1e-4 of each other (both carry the activations at fp32
