@@ -1647,6 +1647,10 @@ struct BatchScratch {
   QScratch q;       // grouped GEMM buffers (MFMA path)
 };
 
+// The grouped GEMMs from two tokens on: with the planes of few tokens packed
+// into one MFMA operand they take 96 against 102 us at 2 tokens, 154 / 187 at
+// 5, 199 / 275 at 8 and 264 / 376 at 12 (K = 8, Q4_K down; Q6_K 112 / 114,
+// 180 / 217, 235 / 325, 305 / 449; K = 4 and 16 alike), and 79 / 69 at one.
 bool batch_uses_mfma(int T) {
   return g_batch_mode == FDM_BATCH_MFMA || (g_batch_mode == FDM_BATCH_AUTO && T >= FDM_BATCH_MFMA_MIN_T);
 }

@@ -332,14 +332,14 @@ int fdm_moe_forward_batched_noalloc(int L, const float *d_X, const float *d_H_in
  * reference; a tuning and test switch).  FDM_BATCH_DOT4: per-token int8
  * digit dot products, each expert tile held in registers while its tokens
  * stream through LDS.  FDM_BATCH_MFMA: the grouped GEMMs on MFMA (exact
- * integer weights 1024 + sc*q in fp16, the activations as three fp16
- * planes: fp32 grade).  FDM_BATCH_AUTO: MFMA from FDM_BATCH_MFMA_MIN_T
- * tokens per step, DOT4 below.  Stores the previous mode in *prev when prev
+ * integer weights in fp16, the activations as three fp16 planes: fp32
+ * grade).  FDM_BATCH_AUTO: MFMA from FDM_BATCH_MFMA_MIN_T tokens per step,
+ * DOT4 below.  Stores the previous mode in *prev when prev
  * is not NULL. */
 #define FDM_BATCH_AUTO 0
 #define FDM_BATCH_DOT4 1
 #define FDM_BATCH_MFMA 2
-#define FDM_BATCH_MFMA_MIN_T 12
+#define FDM_BATCH_MFMA_MIN_T 2
 int fdm_set_batch_kernel(int mode, int *prev);
 
 /* ---- rms_norm on the device (infer.m:369-374, the h_post of infer.m:1850):
