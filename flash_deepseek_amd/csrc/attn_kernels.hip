@@ -12,7 +12,7 @@
 //   c_kv[len] = rms_norm(kv_a[:512] * inv, kv_a_norm); YaRN RoPE of q_rope
 //     and k_rope at pos into k_rope[len]; Q_abs[h] = k_b[h] . q_nope[h]
 //     [128][512]                                            k_mla_prep (one launch)
-//   per 64-position chunk c and 16 heads: scores = scale (Q_abs[h].c_kv[s]
+//   per chunk c of 16, 32 or 64 positions and 16 heads: scores = scale (Q_abs[h].c_kv[s]
 //     + q_rope[h].k_rope[s]), the chunk's max m_c, p = exp(score - m_c),
 //     l_c = sum p, part_c[h] = sum_s p c_kv[s]       k_mla_attn_part
 //   wc[h] = sum_c e^(m_c - M) part_c[h] / sum_c e^(m_c - M) l_c (the softmax
@@ -32,7 +32,7 @@ constexpr int kMvChunk = 512;   // halves per wave load
 constexpr int kMvBatch = 8;     // loads in flight per wave
 constexpr int kMvWaves = 4;
 constexpr int kMvMaxCols = 16384;  // o_proj input: 128 heads x 128
-constexpr int kMvWideWaves = 6;    // waves per workgroup for rows wider than 8192 (o_proj)
+constexpr int kMvWideWaves = 7;    // waves per workgroup for rows wider than 8192 (o_proj)
 
 __device__ __forceinline__ float mv_dot8(u32x4 w, const float* x, float acc) {
   const f32x4 x0 = *reinterpret_cast<const f32x4*>(x), x1 = *reinterpret_cast<const f32x4*>(x + 4);
@@ -67,23 +67,33 @@ __global__ __launch_bounds__(WV * 64) void k_mv_f16(const uint16_t* __restrict__
                                                     const float* __restrict__ res, float* __restrict__ y, int rows,
                                                     int cols) {
   extern __shared__ float xs[];  // cols floats
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n_waves = gridDim.x * WV, chunks = cols / kMvChunk;
+  u32x4 w[NB];
+  auto load = [&](int i, int r, int c) {  // chunk c of row r into slot i
+    w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(W + (size_t)r * cols + 8 * lane + c * kMvChunk));
+  };
+  const int r0 = blockIdx.x * WV + wave;
+  // the first row's first loads before x is staged; later each slot is
+  // refilled as it is used (the row's chunk NB ahead, or the next row's), so
+  // the stream never stops
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+    if (i < chunks && r0 < rows) load(i, r0, i);
+  __builtin_amdgcn_sched_barrier(0);
   for (int i = threadIdx.x; i < cols / 4; i += blockDim.x)
     reinterpret_cast<f32x4*>(xs)[i] = reinterpret_cast<const f32x4*>(x)[i];
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int n_waves = gridDim.x * WV, chunks = cols / kMvChunk;
-  for (int r = blockIdx.x * WV + wave; r < rows; r += n_waves) {
-    const uint16_t* wr = W + (size_t)r * cols + 8 * lane;
+  for (int r = r0; r < rows; r += n_waves) {
     float acc = 0.0f;
     for (int b = 0; b < chunks; b += NB) {
-      u32x4 w[NB];
+      const bool same = b + NB < chunks;
+      const int rn = same ? r : r + n_waves, cn = same ? b + NB : 0;
 #pragma unroll
-      for (int i = 0; i < NB; ++i)
-        if (b + i < chunks) w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wr + (b + i) * kMvChunk));
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < NB; ++i)
+      for (int i = 0; i < NB; ++i) {
         if (b + i < chunks) acc = mv_dot8(w[i], xs + (b + i) * kMvChunk + 8 * lane, acc);
+        if (rn < rows && cn + i < chunks) load(i, rn, cn + i);
+      }
     }
     acc = wave_sum_lane0(acc);  // the butterfly's lane-0 sum, VALU only
     if (lane == 0) y[r] = (res ? res[r] : 0.0f) + acc;
@@ -536,12 +546,14 @@ hipError_t launch_mv_f16(const uint16_t* W, const float* x, const float* res, fl
   const size_t lds = (size_t)cols * sizeof(float);
   const int per_cu = max(1, min(8, (int)((160u << 10) / lds)));  // workgroups per CU the LDS allows
   if (cols > 8192) {
-    // o_proj: 64 KB of x allow two workgroups per CU; six waves each share
-    // it (measured 97.0-97.3 against 97.6-97.7 us per token with four; five,
-    // seven, or sixteen loads in flight no better)
+    // o_proj: 64 KB of x allow two workgroups per CU; seven waves each share
+    // it and have two of the 7168 rows each on 256 CUs, with sixteen loads in
+    // flight: 38.4-38.9 us (6.1 TB/s) against 40.7 with eight, 40.8 with five
+    // waves and 44.4 with eight waves (a third of them a third row), 40.6
+    // before the loads ran ahead of x's staging and across rows
     constexpr int WV = kMvWideWaves;
     const int wgs = min((rows + WV - 1) / WV, per_cu * g_num_cus);
-    k_mv_f16<WV, kMvBatch><<<wgs, WV * 64, lds, s>>>(W, x, res, y, rows, cols);
+    k_mv_f16<WV, 2 * kMvBatch><<<wgs, WV * 64, lds, s>>>(W, x, res, y, rows, cols);
   } else {
     const int wgs = min((rows + kMvWaves - 1) / kMvWaves, per_cu * g_num_cus);
     k_mv_f16<kMvWaves, kMvBatch><<<wgs, kMvWaves * 64, lds, s>>>(W, x, res, y, rows, cols);
@@ -567,6 +579,22 @@ hipError_t launch_mv_f16_rn(const uint16_t* W, const float* x, const float* xmul
   return hipGetLastError();
 }
 
+// A chunk's workgroups read its rows and their heads' queries through one
+// CU's L1 each, which sets the attention's time at few positions, while more
+// chunks make the merge longer.  Both launches, at chunks of 16 / 32 / 64:
+//   S ~ 25: 12.6 / 14.7 / 18.9 us   100: 13.5 / 15.1 / 20.3   200: 15.4 / 16.3 / 20.8
+//   S ~ 400: 18.1 / 18.2 / 21.9     800: 25 / 20.6 / 23.5     1500: 36 / 30 / 25.8
+// (up to 32 chunks are merged with every load issued at dispatch).
+constexpr int kMla16 = 256, kMla32 = 1024;
+int mla_chunk_pos(int S) { return S <= kMla16 ? 16 : S <= kMla32 ? 32 : 64; }
+int mla_chunks(int S) { return (S + mla_chunk_pos(S) - 1) / mla_chunk_pos(S); }
+int mla_max_chunks(int max_seq) {
+  int m = mla_chunks(max_seq);
+  for (int s : {kMla16, kMla32})
+    if (s < max_seq) m = max(m, mla_chunks(s));
+  return m;
+}
+
 hipError_t launch_mla_attend(const MlaArgs& a, hipStream_t s) {
   // RoPE + append, and Q_abs[h] = k_b[h] (512 x 128) . q_nope[h]: 16 lanes
   // per row, 4 rows per wave step, up to 4 workgroups per CU
@@ -578,10 +606,19 @@ hipError_t launch_mla_attend(const MlaArgs& a, hipStream_t s) {
     if (hipError_t e = hipGetLastError()) return e;
   }
   const int S = a.len + 1;
-  const int n_chunks = (S + kMlaChunkPos - 1) / kMlaChunkPos;
+  const int n_chunks = mla_chunks(S);
   if (n_chunks > 1024) return hipErrorInvalidValue;  // k_mla_combine_vb holds <= 1024 chunk weights
-  k_mla_attn_part<kMlaChunkPos><<<dim3(n_chunks, 128 / 16), 512, 0, s>>>(a.q_abs, a.q, a.cache_c, a.cache_k, S,
-                                                                         a.scale, a.part, a.stat);
+  const dim3 grid(n_chunks, 128 / 16);
+  switch (mla_chunk_pos(S)) {
+    case 16:
+      k_mla_attn_part<16><<<grid, 512, 0, s>>>(a.q_abs, a.q, a.cache_c, a.cache_k, S, a.scale, a.part, a.stat);
+      break;
+    case 32:
+      k_mla_attn_part<32><<<grid, 512, 0, s>>>(a.q_abs, a.q, a.cache_c, a.cache_k, S, a.scale, a.part, a.stat);
+      break;
+    default:
+      k_mla_attn_part<64><<<grid, 512, 0, s>>>(a.q_abs, a.q, a.cache_c, a.cache_k, S, a.scale, a.part, a.stat);
+  }
   if (hipError_t e = hipGetLastError()) return e;
   if (n_chunks <= 16)
     k_mla_combine_vb<16><<<128 * 4, 256, 0, s>>>(a.part, a.stat, n_chunks, a.v_b, a.wc, a.attn);

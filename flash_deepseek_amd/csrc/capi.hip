@@ -1975,7 +1975,7 @@ static int ensure_attn(Workspace& w, int seq, hipStream_t s) {
   FDM_HIP(hipStreamSynchronize(s));
   ws.release();
   const size_t H = FDM_HIDDEN, QA = 1536, QB = 128 * 192, KVA = 576, O = 128 * 128;
-  const size_t chunks = (size_t)((seq + kMlaChunkPos - 1) / kMlaChunkPos);
+  const size_t chunks = (size_t)mla_max_chunks(seq);
   // normed[0]: the attention norm's 1 / rms (the rest of H is spare)
   const size_t n[] = {H, QA + KVA, QB, 128 * 512, 128 * 512, O, chunks * 128 * 512, chunks * 128 * 2};
   float** p[] = {&ws.normed, &ws.q_a, &ws.q, &ws.q_abs, &ws.wc, &ws.attn, &ws.part, &ws.stat};

@@ -272,7 +272,12 @@ hipError_t launch_transpose_heads(const uint16_t* src, size_t head_stride, uint1
                                   int cols, hipStream_t s);
 
 // attn_kernels.hip: MLA attention of one decode token
-constexpr int kMlaChunkPos = 64;  // cache positions per attention chunk (16 or 32 or 64)
+// Cache positions per attention chunk at a cache of S positions (64, 32 or
+// 16), the number of chunks, and the largest number at any cache of up to
+// max_seq positions (attn_kernels.hip).
+int mla_chunk_pos(int S);
+int mla_chunks(int S);
+int mla_max_chunks(int max_seq);
 struct MlaArgs {
   float* q;              // [128][192] (q_b output; the rope part rotated in place)
   const float* kv_a;     // [576]: latent (512) + k_rope (64), before RoPE, times *kv_scale
@@ -283,8 +288,8 @@ struct MlaArgs {
   float *cache_c, *cache_k;  // [max_seq][512], [max_seq][64]
   const uint16_t *k_b, *v_b;  // F16 [128][512][128], [128][128][512]
   float *q_abs, *wc, *attn;  // [128][512], [128][512], [128][128]
-  float* part;                        // [ceil(S / kMlaChunkPos)][128][512] partial latent sums
-  float* stat;                        // [ceil(S / kMlaChunkPos)][128][2]: each chunk's max score and exp sum
+  float* part;                        // [mla_chunks(S)][128][512] partial latent sums
+  float* stat;                        // [mla_chunks(S)][128][2]: each chunk's max score and exp sum
   float scale;
 };
 // y[r] = (res ? res[r] : 0) + W[r] . x; cols % 512 == 0, cols <= 16384

@@ -82,6 +82,34 @@ def test_attn_long_cache_matches_oracle(fdm, oracle):
         fdm.attn_release(5)
 
 
+@pytest.mark.parametrize("max_seq", [17, 258, 1026])
+def test_attn_chunk_edges(fdm, oracle, max_seq):
+    """The chunk length of the attention changes at caches of 256 and 1024
+    positions: the last cache of one length, the first of the next, and full
+    and one-position last chunks, in a scratch sized for just that cache."""
+    w = mla_weights(830)
+    say(f"attn_upload L=6 max_seq={max_seq}")
+    fdm.attn_upload(6, w, max_seq=max_seq)
+    try:
+        cache = oracle.MlaCache(max_seq)
+        rng = np.random.default_rng(max_seq)
+        checks = {0, 15, 16, 255, 256, 257, 1023, 1024, 1025}
+        for n in range(max_seq):
+            hidden = rng.normal(0, 1, H).astype(np.float32)
+            d = to_dev(hidden)
+            if n in checks:
+                say(f"attn_forward L=6 pos={n}")
+            fdm.attn_forward(6, d, n)
+            if n in checks:
+                want = oracle.mla_forward(w, hidden, cache, n)
+                err = rel_l2(to_host(d).astype(np.float64) - hidden, want.astype(np.float64) - hidden)
+                assert err <= 1e-5, (n, err)
+            else:
+                oracle.mla_append(w, hidden, cache, n)
+    finally:
+        fdm.attn_release(6)
+
+
 def test_attn_errors(fdm, attn_layer):
     x = to_dev(np.zeros(H, np.float32))
     with pytest.raises(fdm.FdmError):
