@@ -27,7 +27,7 @@ constexpr int kGuChunks = kHidden / kDnChunk;  // 14 per gate/up row
 constexpr int kGuBatch = 7;                    // loads per matrix in flight per wave
 constexpr int kGuWaves = 6;                    // gate/up: 6 waves, 4 workgroups per CU
 constexpr int kDnWaves = 7;                    // down: 7 waves, 2 workgroups per CU
-constexpr int kDnBatch = 12;                   // down loads in flight per wave
+constexpr int kDnBatch = 12;                   // down loads in flight per wave (18: no faster)
 static_assert(kGuChunks % kGuBatch == 0, "gate/up batches tile a row");
 
 // IEEE binary32 -> binary16, round to nearest even, by integer construction:
@@ -136,25 +136,35 @@ __global__ __launch_bounds__(kDnWaves * 64) void k_dense_down(const uint16_t* __
                                                               const float* __restrict__ h_in,
                                                               float* __restrict__ out, int inter) {
   __shared__ float as[kDenseMaxFfn];  // 72 KB
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n_waves = gridDim.x * kDnWaves, chunks = inter / kDnChunk;
+  const int r0 = blockIdx.x * kDnWaves + wave;
+  u32x4 w[kDnBatch];
+  auto load = [&](int i, int r, int c) {  // chunk c of row r into slot i
+    w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(down + (size_t)r * inter + 8 * lane + c * kDnChunk));
+  };
+  // the first row's first loads before the activations are staged; later
+  // each slot is refilled as it is used (the row's chunk kDnBatch ahead, or
+  // the next row's)
+#pragma unroll
+  for (int i = 0; i < kDnBatch; ++i)
+    if (i < chunks && r0 < kHidden) load(i, r0, i);
+  __builtin_amdgcn_sched_barrier(0);
   for (int i = threadIdx.x; i < inter / 4; i += blockDim.x)
     reinterpret_cast<f32x4*>(as)[i] = reinterpret_cast<const f32x4*>(act)[i];
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int n_waves = gridDim.x * kDnWaves, chunks = inter / kDnChunk;
-  for (int r = blockIdx.x * kDnWaves + wave; r < kHidden; r += n_waves) {
-    const uint16_t* dr = down + (size_t)r * inter + 8 * lane;
+  for (int r = r0; r < kHidden; r += n_waves) {
     float d = 0.0f;
     for (int b = 0; b < chunks; b += kDnBatch) {
-      u32x4 w[kDnBatch];
-#pragma unroll
-      for (int i = 0; i < kDnBatch; ++i)
-        if (b + i < chunks) w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(dr + (b + i) * kDnChunk));
+      const bool same = b + kDnBatch < chunks;
+      const int rn = same ? r : r + n_waves, cn = same ? b + kDnBatch : 0;
 #pragma unroll
       for (int i = 0; i < kDnBatch; ++i) {
         if (b + i < chunks) {
           const float* ap = as + (b + i) * kDnChunk + 8 * lane;
           d = dot8(w[i], *reinterpret_cast<const f32x4*>(ap), *reinterpret_cast<const f32x4*>(ap + 4), d);
         }
+        if (rn < kHidden && cn + i < chunks) load(i, rn, cn + i);
       }
     }
     d = wave_sum(d);
