@@ -284,10 +284,20 @@ __device__ __forceinline__ f32x4 mfma_f32x4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// One 16-byte direct global -> LDS load per lane (lane i writes dst + 16 i).
+__device__ __forceinline__ void lds_copy16(const float* src, f32x4* dst) {
+  __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
+}
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // ---- scores, softmax and the weighted latent sum in one pass ----------------------------
 // Flash-decoding over chunks of POS cache positions (infer.m:829-867, the
 // softmax of 385-389 taken apart per chunk and put back together exactly as
 // a rescaled sum).  One workgroup of 8 waves per (chunk c, 16 heads):
+//   0. the chunk's latent rows into LDS (direct loads of whole lines), for
+//      both uses (read from memory by the MFMA lanes a score load touched 16
+//      rows and a sum load took 4 bytes per lane: chunks of 16 / 32 / 64
+//      positions 6.5 / 11.1 / 16.3 -> 5.6 / 10.5 / 15.6 us);
 //   1. scores of its 16 heads x POS positions on fp32 MFMA (16 x 16 tiles;
 //      the 512 latent dims of a tile split over 8 / (POS / 16) waves, whose
 //      partial sums are added in split order; the rope dims by the last
@@ -295,13 +305,13 @@ __device__ __forceinline__ f32x4 mfma_f32x4(float a, float b, f32x4 c) {
 //      two sgemm calls' sum) into LDS;
 //   2. per head: the chunk's max m_c, p = exp(score - m_c), l_c = sum p;
 //   3. part[c][h][d] = sum_s p[h][s] c_kv[s][d] over the chunk on fp32 MFMA
-//      (heads as rows, 16 latent dims per tile, 4 tiles per wave, their
-//      loads issued before the MFMAs),
+//      (heads as rows, 16 latent dims per tile, 4 tiles per wave),
 // and writes (m_c, l_c) for each head.  k_mla_combine_vb then merges the
-// chunks: wc = sum_c exp(m_c - M) part_c / sum_c exp(m_c - M) l_c.  Every
-// stage's loads are in flight at once, so a workgroup pays about one load
-// latency per stage; the chunk length sets how many workgroups share the
-// cache (S / POS x 8).  (Splitting the 512 dims over four workgroups, each
+// chunks: wc = sum_c exp(m_c - M) part_c / sum_c exp(m_c - M) l_c.  All
+// loads are in flight at once, so a workgroup pays about one load latency;
+// then the fp32 MFMAs (32 cycles each, 128 per wave at 64 positions) bound
+// it.  The chunk length sets how many workgroups share the cache
+// (S / POS x 8).  (Splitting the 512 dims over four workgroups, each
 // recomputing the chunk's scores, measured slower: the scores' latent reads
 // quadruple.)
 template <int POS>
@@ -313,6 +323,10 @@ __global__ __launch_bounds__(512) void k_mla_attn_part(const float* __restrict__
   constexpr int KS = 8 / PT;    // latent splits per tile
   constexpr int MS = 32 / KS;   // 16-dim steps per split
   static_assert(PT * KS == 8 && MS * KS == 32, "8 waves cover the tiles and splits");
+  // the chunk's latent rows: 128 pieces of 16 bytes, piece p of row s at
+  // p ^ (s % 16), so that both a column of 16 rows (scores) and a run of 16
+  // pieces of one row (weighted sum) read distinct banks
+  __shared__ __attribute__((aligned(16))) f32x4 cs[POS * 128];
   __shared__ float sp[KS][16][POS + 1];  // latent partial scores per split (row = head)
   __shared__ float sr[16][POS + 1];      // rope scores
   __shared__ float ps[16][POS + 1];      // p
@@ -327,15 +341,11 @@ __global__ __launch_bounds__(512) void k_mla_attn_part(const float* __restrict__
     const int s0 = base + 16 * tile;
     const int sp_row = min(s0 + r, S - 1);  // past the cache: a valid row, result not kept
     const float* qa = q_abs + (size_t)(h0 + r) * 512 + 16 * MS * ks + 4 * q4;
-    const float* cc = cache_c + (size_t)sp_row * 512 + 16 * MS * ks + 4 * q4;
     const float* qr = q + (size_t)(h0 + r) * 192 + 128 + 4 * q4;
     const float* kr = cache_k + (size_t)sp_row * 64 + 4 * q4;
-    f32x4 x[MS], y[MS], kx[4], ky[4];
+    f32x4 x[MS], kx[4], ky[4];
 #pragma unroll
-    for (int m = 0; m < MS; ++m) {
-      x[m] = *reinterpret_cast<const f32x4*>(qa + 16 * m);
-      y[m] = *reinterpret_cast<const f32x4*>(cc + 16 * m);
-    }
+    for (int m = 0; m < MS; ++m) x[m] = *reinterpret_cast<const f32x4*>(qa + 16 * m);
     if (rope) {
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
@@ -343,14 +353,25 @@ __global__ __launch_bounds__(512) void k_mla_attn_part(const float* __restrict__
         ky[m] = *reinterpret_cast<const f32x4*>(kr + 16 * m);
       }
     }
-    __builtin_amdgcn_sched_barrier(0);
+    // wave w copies half rows w, w + 8, ..: 64 pieces each, one direct
+    // global -> LDS load (rows past the cache: the last row, against p = 0)
+#pragma unroll
+    for (int k = 0; k < POS / 4; ++k) {
+      const int half = wave + 8 * k, row = half >> 1, p0 = 64 * (half & 1);
+      const int piece = (p0 + lane) ^ (row & 15);
+      lds_copy16(cache_c + (size_t)min(base + row, S - 1) * 512 + 4 * piece, &cs[row * 128 + p0]);
+    }
+    wait_loads();
+    __syncthreads();
     f32x4 a[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) a[e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int m = 0; m < MS; ++m)
+    for (int m = 0; m < MS; ++m) {
+      const f32x4 y = cs[(16 * tile + r) * 128 + ((4 * (MS * ks + m) + q4) ^ r)];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) a[e] = mfma_f32x4(x[m][e], y[m][e], a[e]);
+      for (int e = 0; e < 4; ++e) a[e] = mfma_f32x4(x[m][e], y[e], a[e]);
+    }
     // D: lane l holds heads 4 (l / 16) + v, position s0 + l % 16
 #pragma unroll
     for (int v = 0; v < 4; ++v) sp[ks][4 * q4 + v][16 * tile + r] = (a[0][v] + a[1][v]) + (a[2][v] + a[3][v]);
@@ -400,36 +421,29 @@ __global__ __launch_bounds__(512) void k_mla_attn_part(const float* __restrict__
     }
   }
   __syncthreads();
-  // 3. the chunk's weighted latent sums: wave w takes dim tiles w, w + 8,
-  //    w + 16, w + 24 (step e of a group of 16 positions takes from lane l
-  //    the position 16 g + 4 (l / 16) + e).  Positions past the cache read
-  //    the last row (finite) against p = 0.
-  float y[4][PT][4];
+  // 3. the chunk's weighted latent sums: wave w takes dims 64 w .. 64 w + 63,
+  //    column r of its tile i dim 64 w + 4 r + i, so a lane's one 16-byte read
+  //    of position 4 g + q4 serves four tiles; the groups g are summed in
+  //    four chains.
+  f32x4 acc[4][4];  // [tile][chain]
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d0 = 16 * (wave + 8 * i);
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int g = 0; g < PT; ++g)
+    for (int e = 0; e < 4; ++e) acc[i][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int sidx = min(base + 16 * g + 4 * q4 + e, S - 1);
-        y[i][g][e] = cache_c[(size_t)sidx * 512 + d0 + r];
-      }
+  for (int g = 0; g < POS / 4; ++g) {
+    const int row = 4 * g + q4;
+    const f32x4 y = cs[row * 128 + ((16 * wave + r) ^ (row & 15))];
+    const float p = ps[r][row];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i][g & 3] = mfma_f32x4(p, y[i], acc[i][g & 3]);
   }
-  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int d0 = 16 * (wave + 8 * i);
-    f32x4 acc[4];
+  for (int v = 0; v < 4; ++v) {
+    f32x4 o;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int g = 0; g < PT; ++g)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] = mfma_f32x4(ps[r][16 * g + 4 * q4 + e], y[i][g][e], acc[e]);
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-      part[((size_t)c * 128 + h0 + 4 * q4 + v) * 512 + d0 + r] = (acc[0][v] + acc[1][v]) + (acc[2][v] + acc[3][v]);
+    for (int i = 0; i < 4; ++i) o[i] = (acc[i][0][v] + acc[i][1][v]) + (acc[i][2][v] + acc[i][3][v]);
+    *reinterpret_cast<f32x4*>(part + ((size_t)c * 128 + h0 + 4 * q4 + v) * 512 + 64 * wave + 4 * r) = o;
   }
 }
 
@@ -579,11 +593,11 @@ hipError_t launch_mv_f16_rn(const uint16_t* W, const float* x, const float* xmul
   return hipGetLastError();
 }
 
-// A chunk's workgroups read its rows and their heads' queries through one
-// CU's L1 each, which sets the attention's time at few positions, while more
-// chunks make the merge longer.  Both launches, at chunks of 16 / 32 / 64:
-//   S ~ 25: 12.6 / 14.7 / 18.9 us   100: 13.5 / 15.1 / 20.3   200: 15.4 / 16.3 / 20.8
-//   S ~ 400: 18.1 / 18.2 / 21.9     800: 25 / 20.6 / 23.5     1500: 36 / 30 / 25.8
+// A chunk is a workgroup's work for its 16 heads, so short chunks spread few
+// positions over more CUs, while more chunks make the merge longer.  Both
+// launches, at chunks of 16 / 32 / 64:
+//   S ~ 25: 11.9 / 13.9 / 18.4 us   100: 12.9 / 14.3 / 18.7   200: 14.9 / 15.4 / 19.0
+//   S ~ 400: 17.9 / 17.2 / 20.2     800: 25.0 / 20.2 / 22.4   1200: 30.7 / 26.7 / 24.0
 // (up to 32 chunks are merged with every load issued at dispatch).
 constexpr int kMla16 = 256, kMla32 = 1024;
 int mla_chunk_pos(int S) { return S <= kMla16 ? 16 : S <= kMla32 ? 32 : 64; }
