@@ -83,8 +83,9 @@ __global__ __launch_bounds__(256) void k_dequant_q6k(const uint8_t* __restrict__
 // block's header and its 8 half-groups go to their REL places (rel_step_off /
 // rel_piece).  Consecutive threads take the rows of a step, then its blocks,
 // then the next step, so 16 threads write four whole 64-byte runs per store
-// and read four runs of 576 B (one thread per block in the matrix's own order
-// wrote 16 bytes to each line: 6.6 GB of a layer took 6.4 instead of 4.1 ms).
+// and read four runs of 576 B: 2.9 ms for the 6.3 GB of a layer (4.4 TB/s read
+// and written; one thread per block in the matrix's own order wrote 16 bytes
+// to each line and made an attach 2.4 ms longer).
 // Blob b of n: src + b * src_stride -> dst + b * expert_size.  A Q6_K down
 // matrix goes through k_rel_pack_q6.
 __global__ __launch_bounds__(256) void k_rel_pack(const uint8_t* __restrict__ src, size_t src_stride,
