@@ -125,13 +125,23 @@ __global__ __launch_bounds__(256) void k_route(const float* __restrict__ logits,
   route_wave(logits + (size_t)t * 256, bias, K, 2.5f, idx + (size_t)t * K, w + (size_t)t * K);
 }
 
+// The batched logits are bound by the latency and the L2 traffic of their
+// loads.  Blocks of 4 x 4 give n_exp / 4 workgroups per 4 tokens, so a few
+// tokens still fill the chip; blocks of 8 x 8 read half as much per logit,
+// which counts once the blocks are many.  Measured at 256 experts of 7168
+// (4 x 4 against the path before, us): T = 2: 6.4 / 6.8, 8: 7.1 / 17.3 (one
+// expert x 8 tokens), 16: 8.6 / 14.5, 32: 11.0 / 16.2, 48: 14.2 / 16.6,
+// 64: 17.6 / 16.6, 128: 28.4 / 22.6 (8 x 8); hence the line at 48.
 hipError_t launch_router_logits(const float* Wg, const float* x, int n_exp, int dim, int T,
                                 float* logits, hipStream_t s) {
   if (T <= 1) {
     hipLaunchKernelGGL(k_router_logits<1>, dim3(n_exp, T), dim3(256), 0, s, Wg, x, n_exp, dim,
                        T, logits);
-  } else if (T >= 16 && n_exp % 8 == 0) {
+  } else if (T > 48 && n_exp % 8 == 0) {
     hipLaunchKernelGGL((k_router_logits_blk<8, 8>), dim3(n_exp / 8, (T + 7) / 8), dim3(256), 0, s, Wg, x,
+                       n_exp, dim, T, logits);
+  } else if (T <= 48 && n_exp % 4 == 0) {
+    hipLaunchKernelGGL((k_router_logits_blk<4, 4>), dim3(n_exp / 4, (T + 3) / 4), dim3(256), 0, s, Wg, x,
                        n_exp, dim, T, logits);
   } else {
     hipLaunchKernelGGL(k_router_logits<8>, dim3(n_exp, (T + 7) / 8), dim3(256), 0, s, Wg, x,

@@ -31,6 +31,22 @@ def test_router_logits_bit_exact(fdm, oracle, T):
         assert np.array_equal(got[t].view(np.uint32), oracle.router_logits(Wg, X[t]).view(np.uint32))
 
 
+@pytest.mark.parametrize("T,n_exp,dim", [(2, 256, 7168), (3, 256, 7168), (4, 8, 1028), (7, 12, 516), (16, 256, 7168),
+                                         (47, 12, 2048), (48, 256, 7168), (49, 256, 7168), (49, 12, 516),
+                                         (5, 6, 1028), (50, 6, 516)])
+def test_router_logits_block_edges(fdm, oracle, T, n_exp, dim):
+    """Both sides of the rule between blocks of 4 x 4 and 8 x 8, blocks with
+    tokens past the end, and expert counts that fit neither; bit-exact."""
+    say(f"router_logits T={T} n_exp={n_exp} dim={dim}")
+    Wg = oracle.synth_normal(n_exp * dim, 0.0, 0.01, 50).reshape(n_exp, dim)
+    X = oracle.synth_normal(T * dim, 0.0, 1.0, 51 + T).reshape(T, dim)
+    out = empty_f32(T * n_exp)
+    fdm.router_logits(to_dev(Wg), to_dev(X), out, T=T)
+    got = to_host(out).reshape(T, n_exp)
+    for t in range(T):
+        assert np.array_equal(got[t].view(np.uint32), oracle.router_logits(Wg, X[t]).view(np.uint32))
+
+
 @pytest.mark.parametrize("K", [1, 4, 8, 16])
 def test_route_bit_exact_random(fdm, oracle, K):
     T = 300
