@@ -1505,14 +1505,11 @@ QScratch workspace_q(const Workspace& w) {
   return QScratch{w.q_planes, w.q_xs, w.q_xe, w.q_chunks, w.q_nchunks};
 }
 
-// The expert half of one step on the grouped GEMMs, after the dispatch:
-// chunk list, planes of the token rows (unless x_planes_ready: the caller
-// has written them), gate/up + SwiGLU into b.act, the planes of b.act and the
-// down into b.eo.  A Q6_K down takes three planes always, in chunks of their
+// The expert half of one step on the grouped GEMMs, on the planes of the
+// token rows that the caller has written: dispatch with the chunk list,
+// gate/up + SwiGLU into b.act, the planes of b.act and the down into b.eo.  A Q6_K down takes three planes always, in chunks of their
 // size (one-plane callers have a second chunk list for it in the workspace).
-// x: the fp32 token rows [T][7168].
-int run_qgemm_experts(const Layer* y, const BatchArgs& b0, const float* x, int planes, const QScratch& w,
-                      hipStream_t s, bool x_planes_ready = false) {
+int run_qgemm_experts(const Layer* y, const BatchArgs& b0, int planes, const QScratch& w, hipStream_t s) {
   BatchArgs b = b0;
   const int T = b.T, K = b.K;
   const size_t rows = (size_t)T * K + (y->shared ? T : 0);
@@ -1533,7 +1530,6 @@ int run_qgemm_experts(const Layer* y, const BatchArgs& b0, const float* x, int p
     if (mc_down > kQMaxChunks) return fail(FDM_E_INVAL, "chunk list of %d entries exceeds %d", mc_down, kQMaxChunks);
   }
   FDM_HIP(launch_dispatch(b, s));  // with the chunk lists
-  if (!x_planes_ready) FDM_HIP(launch_xplanes(x, FDM_HIDDEN, (size_t)T, planes, w.planes, w.xs, w.xe, s));
   QGemmArgs q;
   q.T = T;
   q.K = K;
@@ -1549,7 +1545,7 @@ int run_qgemm_experts(const Layer* y, const BatchArgs& b0, const float* x, int p
   q.n_chunks = w.n_chunks;
   q.out = b.act;
   FDM_HIP(launch_qgemm(q, planes, false, false, mc, s));
-  FDM_HIP(launch_xplanes(b.act, FDM_MOE_FFN, rows, planes_down, w.planes, w.xs, w.xe, s));
+  FDM_HIP(launch_xplanes(b.act, rows, planes_down, w.planes, w.xs, w.xe, s));
   q.plane = rows * FDM_MOE_FFN;
   q.out = b.eo;
   if (own_list) {
@@ -1620,7 +1616,7 @@ int fdm_moe_prefill(const int* layers, int n_layers, float* d_H, int T, int K,
     b.distinct = w.b_distinct;
     b.n_distinct = w.b_ndistinct;
     // prefill precision: one fp16 plane of the activations (the bar is 1e-2)
-    if (int rc = run_qgemm_experts(y, b, w.p_hpost, 1, workspace_q(w), s, true)) return rc;
+    if (int rc = run_qgemm_experts(y, b, 1, workspace_q(w), s)) return rc;
     FDM_HIP(launch_combine(b, s));
   }
   return FDM_OK;
@@ -1663,7 +1659,11 @@ int batched_step(const Layer* y, const float* d_X, const float* d_H_in, int T, i
   float* w = d_w ? d_w : sc.w;
   ProfScope p(FDM_PROF_BATCH, s);
   FDM_HIP(launch_router_logits(y->Wg, d_X, FDM_N_EXPERTS, FDM_HIDDEN, T, sc.logits, s));
-  FDM_HIP(launch_route(sc.logits, y->bias, T, K, idx, w, s));
+  const bool mfma = batch_uses_mfma(T);
+  if (mfma)
+    FDM_HIP(launch_route_xplanes(sc.logits, y->bias, T, K, idx, w, d_X, sc.q.planes, sc.q.xs, sc.q.xe, s));
+  else
+    FDM_HIP(launch_route(sc.logits, y->bias, T, K, idx, w, s));
   BatchArgs b;
   b.T = T;
   b.K = K;
@@ -1684,12 +1684,12 @@ int batched_step(const Layer* y, const float* d_X, const float* d_H_in, int T, i
   b.pair_of = sc.pair_of;
   b.distinct = sc.distinct;
   b.n_distinct = d_n_distinct ? d_n_distinct : sc.n_distinct;
-  if (!batch_uses_mfma(T)) {
+  if (!mfma) {
     FDM_HIP(launch_batched_experts(b, y->down_q6, s));
     return FDM_OK;
   }
   // grouped MFMA GEMMs at fp32 grade (three fp16 planes of the activations)
-  if (int rc = run_qgemm_experts(y, b, d_X, 3, sc.q, s)) return rc;
+  if (int rc = run_qgemm_experts(y, b, 3, sc.q, s)) return rc;
   FDM_HIP(launch_combine(b, s));
   return FDM_OK;
 }

@@ -222,7 +222,7 @@ hipError_t launch_combine(const BatchArgs& b, hipStream_t s);
 // rms_norm per token (infer.m:369-374), bit-exact: o = x * inv * w.  d <= 7168.
 hipError_t launch_rms_norm(const float* x, const float* w, float* o, int T, int d, hipStream_t s);
 // rms_norm of T tokens of 7168 (o, as launch_rms_norm) and the one-plane
-// activation planes of o for the grouped GEMMs (launch_xplanes, planes = 1).
+// activation planes of o for the grouped GEMMs (as launch_xplanes makes one).
 hipError_t launch_rms_norm_planes(const float* x, const float* w, float* o, int T, _Float16* xp, float* xs,
                                   float* xe, hipStream_t s);
 
@@ -242,10 +242,13 @@ struct QGemmArgs {
   const int* n_chunks;
   float* out;              // gate/up: act [rows][2048] (SwiGLU); down: eo [rows][7168]
 };
-// n_rows x [kd] fp32 -> `planes` (1 or 3) fp16 planes of x * 2^s, the
+// n_rows x [2048] fp32 -> `planes` (1 or 3) fp16 planes of x * 2^s, the
 // sub-block sums and 2^-s per row.
-hipError_t launch_xplanes(const float* x, int kd, size_t n_rows, int planes, _Float16* xp, float* xs, float* xe,
+hipError_t launch_xplanes(const float* x, size_t n_rows, int planes, _Float16* xp, float* xs, float* xe,
                           hipStream_t s);
+// launch_route and the three planes of the T token rows x [T][7168].
+hipError_t launch_route_xplanes(const float* logits, const float* bias, int T, int K, int* idx, float* w,
+                                const float* x, _Float16* xp, float* xs, float* xe, hipStream_t s);
 int qgemm_chunk_tokens(int planes);
 constexpr int kQMaxChunks = 1024;  // >= 256 + 512 * 16 / 16 + 512 / 16
 // Q4_K gate/up + SwiGLU (down = false), or the down, Q4_K or (q6, three planes
