@@ -662,13 +662,19 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   dma(0, 0);
   u32x2 xa[NBX], xb[NBX];
   load_xs(xa, 0);
+  __builtin_amdgcn_sched_barrier(0);
   load_hdr(wb, 1);
   load_q(wb, 1, 0);
   load_q(wb, 1, 1);
+  __builtin_amdgcn_sched_barrier(0);
   // Block b from buffer b & 1 while block b + 1 lands in the other one.  The
   // wait before a block leaves the NLOADS youngest loads in flight (the weights
   // of block b + 1): the loads before them, block b's weights, operands and
-  // sub-block sums, have then landed.
+  // sub-block sums, have then landed.  That holds only in this order of issue,
+  // which the scheduling barriers keep, here and around every refill: a
+  // compiler free to move a weight load ahead of a direct load (its max-ilp
+  // strategy does) would let a wave past the wait with its part of the buffer
+  // still in flight, and the others read the block before.
   auto pair = [&](int b, bool last) {
     wait_vm<NLOADS>();
     __syncthreads();  // block b staged by every wave; buffer 1 read by all (block b - 1)
