@@ -314,6 +314,15 @@ __device__ __forceinline__ void lds_dma16(rsrc_t r, uint32_t lane_off, uint32_t 
                                            (int)off, 0, 0);
 }
 
+// LDS shared by the lanes of one wave: what they wrote before is there for the
+// reads after.  The hardware runs a wave's LDS operations in order; this keeps
+// the compiler, which sees one lane only, from moving them.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // waits until at most N of the wave's loads are in flight
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -739,6 +748,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
           const int r = 16 * nb + 4 * j + i;
           red[r * 16 + c16] = acc[tt][nb][i];
         }
+      wave_lds_fence();  // the values of other lanes are read below
       auto sum = [&](const float* p) { return (p[2 * n * 16] + p[n * 16]) + p[0]; };
       if (writer) {
         for (int t = j; t < n; t += 4) {
@@ -746,7 +756,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
           put(t, tt, sum(p), DOWN ? 0.0f : sum(p + 2));
         }
       }
-      __builtin_amdgcn_wave_barrier();  // the next tile's values overwrite these
+      wave_lds_fence();  // the next tile's values overwrite these
     }
   }
 }

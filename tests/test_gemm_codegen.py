@@ -51,3 +51,22 @@ def test_counted_waits_cover_the_direct_loads(assembly):
                 waits += 1
                 assert not any(re.search(r"\blds\b", x) for x in loads[-int(m[1]):]), (kernel, ln, loads[-int(m[1]):])
     assert waits >= 5 * 3
+
+
+def test_plane_sums_read_after_a_fence(assembly):
+    """The packed bodies add a token's three planes across lanes through LDS:
+    between a tile's LDS writes and the reads of other lanes' values, and again
+    before the next tile's writes, stands a wave barrier (with its fences)."""
+    epilogues = 0
+    for kernel, lines in assembly.items():
+        if "ILi3E" not in kernel:  # three planes
+            continue
+        ops = ""
+        for ln in lines:
+            ops += ("b" if "wave barrier" in ln else "w" if ln.startswith("ds_write") else
+                    "r" if ln.startswith("ds_read") else "S" if re.match(r"(global|buffer)_store", ln) else "")
+        tiles = re.findall(r"w(b*)r+S(b*)", ops)  # a tile's values, the sums over them, the output
+        tiles = [t for t in tiles if t[1]]  # the other bodies store what they hold
+        epilogues += len(tiles)
+        assert tiles and all(t == ("b", "b") for t in tiles), (kernel, ops)
+    assert epilogues >= 3 * 4
