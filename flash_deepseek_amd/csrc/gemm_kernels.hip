@@ -420,7 +420,11 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   constexpr int NBX = (NTOK + 15) / 16;      // 16-row blocks that hold plane 0 rows
   constexpr int ROUNDS = PK * NT16 / (2 * kQWaves);  // direct loads per wave per block (2 rows each)
   static_assert(ROUNDS * 2 * kQWaves == PK * NT16, "the direct loads tile the buffer");
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // the wave's number as a scalar: as a vector value it kept each LDS
+  // destination of the direct loads in a register, and the Q6_K down spilled
+  // 18, reloaded in the contraction behind waits for every load in flight
+  // (a step of 64 tokens 785 -> 768 us, 150 prompt tokens 1086 -> 1070)
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c16 = lane & 15, j = lane >> 4;
   const int n = ck.z;
   const bool shared = ck.x < 0;

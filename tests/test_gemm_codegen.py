@@ -70,3 +70,11 @@ def test_plane_sums_read_after_a_fence(assembly):
         epilogues += len(tiles)
         assert tiles and all(t == ("b", "b") for t in tiles), (kernel, ops)
     assert epilogues >= 3 * 4
+
+
+def test_nothing_spills(assembly):
+    """No GEMM keeps registers in scratch memory: a reload inside the
+    contraction waits for every older load and so drains the weight stream."""
+    for kernel, lines in assembly.items():
+        touched = [ln for ln in lines if ln.startswith("scratch_")]
+        assert not touched, (kernel, len(touched), touched[:3])
