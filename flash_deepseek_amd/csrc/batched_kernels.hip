@@ -113,12 +113,12 @@ __device__ __forceinline__ int block_scan_excl(int v, int* wsum, int& tot) {
 
 // One workgroup, thread e < 256 = expert e: pair counts per expert, segment
 // starts, the ascending list of distinct experts, each pair's position in
-// its expert's segment and, with b.ch > 0, the grouped GEMMs' chunk list (with
-// b.ch_down > 0 a second one for the down GEMM; every distinct expert's segment in chunks of b.ch pairs, ascending, then
-// the shared expert's tokens in chunks of b.ch), all by block-wide scans.
-// Pairs keep their order inside a segment, so that a call's results do not
-// vary from run to run: the grouped GEMMs sum a token's planes in an order
-// that depends on its chunk's size.  Each wave takes a contiguous part of
+// its expert's segment and, with b.ch > 0, the grouped GEMMs' chunk list (every
+// distinct expert's segment in chunks of b.ch pairs, ascending, then the shared
+// expert's tokens in chunks of b.ch; with b.ch_down > 0 a second one for the
+// down GEMM), all by block-wide scans.
+// Pairs keep their order inside a segment: a token is in the same chunk of its
+// expert, and its row in the same place of it, in every run.  Each wave takes a contiguous part of
 // the pairs, counts it per expert, and places it 64 pairs at a time: a pair's
 // position is the wave's next free one of its expert plus its rank among the
 // 64, found by eight ballots (one per bit of the expert id).  The first 64

@@ -48,7 +48,7 @@
 // weights for the operand) and the matrix cores (16 cycles per 16x16x32, 32
 // per 16x16x4) need about as long and overlap only partly, so the kernel
 // lives on loads in flight and on few instructions:
-//  - the three planes of a chunk of few tokens share 16-row operands (PACK):
+//  - the three planes of a chunk of few tokens share 16-row operands:
 //    up to 5 tokens cost 8 MFMAs per tile and block instead of 24 and a
 //    third of the LDS traffic; with that, two tiles per wave and three waves
 //    per SIMD beat four tiles and two waves (16-token step 234 against 279 us);
@@ -172,12 +172,8 @@ __device__ __forceinline__ BPair build_b(uint32_t w0, uint32_t w1, f16x2 k, f16x
 // them, so (0x6400 | q) - 1056 is q - 32 (and (0x6400 | 16 q) - 1536 is
 // 16 (q - 32)) exactly; then one packed multiply and one packed fma for the
 // rest.  Element order inside each 8 as for Q4_K.
-struct BPair6 {
-  f16x8 lo, lo_r, hi, hi_r;
-};
-
 template <bool HIGH>
-__device__ __forceinline__ void q6_pair(uint32_t l, uint32_t h, f16x2 k, uint32_t& v, uint32_t& r) {
+__device__ __forceinline__ void q6_pair(uint32_t l, uint32_t h, _Float16 k1, uint32_t& v, uint32_t& r) {
   uint32_t t;
   if (HIGH) {
     asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(t) : "v"(l), "s"(0x00F000F0u), "v"(0x64006400u));
@@ -188,32 +184,30 @@ __device__ __forceinline__ void q6_pair(uint32_t l, uint32_t h, f16x2 k, uint32_
   }
   const _Float16 off = HIGH ? (_Float16)-1536.0f : (_Float16)-1056.0f;
   const f16x2 e = __builtin_bit_cast(f16x2, t) + (f16x2){off, off};
-  const f16x2 a = e * k;
+  const f16x2 k = {k1, k1}, a = e * k;
   v = __builtin_bit_cast(uint32_t, a);
   r = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(e, k, -a));
 }
 
-// ql dwords w0, w1 and qh dwords h0, h1 of the 8 bytes; SH: the quarter's two
-// qh bits lie at bits 0 (quarters 0 and 2: 0 and 4) or 2 (1 and 3: 2 and 6).
-template <int K>
-__device__ __forceinline__ BPair6 build_b6(uint32_t w0, uint32_t w1, uint32_t h0, uint32_t h1, f16x2 k_lo, f16x2 k_hi) {
-  u32x4 lo, lr, hi, hr;
+// One nibble's operands: ql dwords w0, w1 and qh dwords h0, h1 of the 8 bytes.
+// K = 0: quarters 0 (HIGH: 2), whose two qh bits lie at bits 0 (4) of a byte;
+// K = 1: quarters 1 (3), at bits 2 (6).
+struct BHalf6 {
+  f16x8 v, r;
+};
+template <int K, bool HIGH>
+__device__ __forceinline__ BHalf6 build_b6(uint32_t w0, uint32_t w1, uint32_t h0, uint32_t h1, _Float16 k) {
+  u32x4 bv, br;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const uint32_t w = i ? w1 : w0, h = i ? h1 : h0;
-    const uint32_t he = K ? h << 2 : h << 4, ho = K ? h >> 6 : h >> 4, wo = w >> 8;
     uint32_t v, r;
-    q6_pair<false>(w, he, k_lo, v, r);
-    lo[2 * i] = v, lr[2 * i] = r;
-    q6_pair<false>(wo, ho, k_lo, v, r);
-    lo[2 * i + 1] = v, lr[2 * i + 1] = r;
-    q6_pair<true>(w, he, k_hi, v, r);
-    hi[2 * i] = v, hr[2 * i] = r;
-    q6_pair<true>(wo, ho, k_hi, v, r);
-    hi[2 * i + 1] = v, hr[2 * i + 1] = r;
+    q6_pair<HIGH>(w, K ? h << 2 : h << 4, k, v, r);
+    bv[2 * i] = v, br[2 * i] = r;
+    q6_pair<HIGH>(w >> 8, K ? h >> 6 : h >> 4, k, v, r);
+    bv[2 * i + 1] = v, br[2 * i + 1] = r;
   }
-  return BPair6{__builtin_bit_cast(f16x8, lo), __builtin_bit_cast(f16x8, lr), __builtin_bit_cast(f16x8, hi),
-                __builtin_bit_cast(f16x8, hr)};
+  return BHalf6{__builtin_bit_cast(f16x8, bv), __builtin_bit_cast(f16x8, br)};
 }
 
 // Per-block constants of the lane's row: d and, for each quarter k, the
@@ -221,7 +215,7 @@ __device__ __forceinline__ BPair6 build_b6(uint32_t w0, uint32_t w1, uint32_t h0
 // halves).
 struct QScale6 {
   float d;
-  f16x2 k[4];
+  f16x2 k01, k23;
 };
 
 __device__ __forceinline__ QScale6 qscale6(const QLane<kDownQ6>& w, int s) {
@@ -231,7 +225,7 @@ __device__ __forceinline__ QScale6 qscale6(const QLane<kDownQ6>& w, int s) {
     return __builtin_bit_cast(f16x2, b) + (f16x2){(_Float16)-1152.0f, (_Float16)-1152.0f};
   };
   const f16x2 a = two(w.sc.x), b = two(w.sc.y) * (f16x2){(_Float16)0.0625f, (_Float16)0.0625f};
-  return QScale6{half_to_float(w.d), {(f16x2){a.x, a.x}, (f16x2){a.y, a.y}, (f16x2){b.x, b.x}, (f16x2){b.y, b.y}}};
+  return QScale6{half_to_float(w.d), a, b};
 }
 
 // Per-block constants of the lane's row and group, halves for sub-blocks 2j
@@ -400,26 +394,26 @@ __global__ __launch_bounds__(256) void k_route_xplanes(const float* __restrict__
 
 // ---- the grouped GEMM ------------------------------------------------------------------
 // One chunk (n tokens) of one expert, one row group.  The token operand has
-// PK * 16 NB rows in LDS: with PACK = false row (p, r) is plane p of token r
-// and a token block's PK planes accumulate into one register set; with PACK
-// = true (PK = 1) row r is plane r / n of token r % n, so the three planes
+// 16 NB rows in LDS, row r plane r / n of token r % n, so the three planes
 // of up to 5 (NB = 1) or 10 (NB = 2) tokens share the 16-row operands that
-// padding would otherwise fill, and are added up once after the last block.
+// padding would otherwise fill.  Every row is summed by itself, in the same
+// steps whatever NB and r are, and a token's planes are added up once after
+// the last block: a token's bits do not depend on the others of its chunk.
 // NT: the expert has one chunk, its weights are read once and streamed past
 // the L2.
-template <int P, int PK, int NB, bool PACK, QMat M, bool NT>
+template <int P, int NB, QMat M, bool NT>
 __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, uint8_t* lds1, int* rows, const int4 ck,
                                            int rg) {
-  static_assert(PACK ? PK == 1 && P == 3 : PK == P, "packed rows carry one plane each");
   constexpr int TL = kQTiles;
   constexpr bool DOWN = M != kGateUp, Q6 = M == kDownQ6;
   constexpr int KD = DOWN ? kFfn : kHidden;  // contraction length
   constexpr int NBLK = KD / kQK;             // 8 or 28 (even)
-  constexpr int NT16 = 16 * NB;              // operand rows per plane slot
-  constexpr int NTOK = PACK ? NT16 / 3 : NT16;
+  constexpr int NT16 = 16 * NB;              // operand rows
+  constexpr int NTOK = NT16 / P;
+  constexpr bool TIGHT = P == 3 && NB == 3;  // registers are short
   constexpr int NBX = (NTOK + 15) / 16;      // 16-row blocks that hold plane 0 rows
-  constexpr int ROUNDS = PK * NT16 / (2 * kQWaves);  // direct loads per wave per block (2 rows each)
-  static_assert(ROUNDS * 2 * kQWaves == PK * NT16, "the direct loads tile the buffer");
+  constexpr int ROUNDS = NT16 / (2 * kQWaves);  // direct loads per wave per block (2 rows each)
+  static_assert(ROUNDS * 2 * kQWaves == NT16, "the direct loads tile the buffer");
   // the wave's number as a scalar: as a vector value it kept each LDS
   // destination of the direct loads in a register, and the Q6_K down spilled
   // 18, reloaded in the contraction behind waits for every load in flight
@@ -441,24 +435,24 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   const uint8_t* blob = shared ? g.shared : g.experts + (size_t)ck.x * g.expert_size;
   const uint8_t* mat = blob + (DOWN ? 2 * (size_t)kGateBytes : 0);
   constexpr int ROWS = qgemm_rows(DOWN);
-  uint32_t qoff[TL], hoff[TL], soff[TL];
-  int row[TL];
-#pragma unroll
-  for (int t = 0; t < TL; ++t) {
-    // gate/up: column c16 of tile t is row 2 (4 t + c16 / 4) + c16 % 2 of the
-    // wave's 16, of gate for c16 % 4 < 2, else of up
-    row[t] = DOWN ? rg * ROWS + 16 * TL * wave + 16 * t + c16
-                  : rg * ROWS + 8 * TL * wave + 8 * t + 2 * (c16 >> 2) + (c16 & 1);
-    if constexpr (Q6) {
-      const uint32_t base = (uint32_t)rel6_step_off(row[t], 0), bi = (uint32_t)rel6_block_index(row[t], 0);
-      qoff[t] = base + 16 * (2 * bi + (j >> 1)) + 2048 * (j & 1);
-      soff[t] = base + 16 * bi + 8 * (j >> 1);
-      hoff[t] = base + 2 * bi;
-    } else {
-      const uint32_t base = (uint32_t)rel_step_off<DOWN>(row[t], 0), ri = c16 & 3;
-      qoff[t] = base + 16 * (uint32_t)rel_piece((int)ri, 0, j);
-      hoff[t] = base + kRelHdr + 16 * ri;
-    }
+  // gate/up: column c16 of tile t is row 2 (4 t + c16 / 4) + c16 % 2 of the
+  // wave's 16, of gate for c16 % 4 < 2, else of up.  Tile t's rows lie t
+  // kTileRows further and its bytes t kTileStep: a scalar offset, so that a lane
+  // keeps the addresses of tile 0 only.
+  constexpr int kTileRows = DOWN ? 16 : 8;
+  constexpr uint32_t kTileStep = Q6 ? kRel6Step : kRelStep * (DOWN ? 4 : 4 * (kHidden / 1024));
+  const int row0 = DOWN ? rg * ROWS + 16 * TL * wave + c16
+                        : rg * ROWS + 8 * TL * wave + 2 * (c16 >> 2) + (c16 & 1);
+  uint32_t qoff, hoff, soff = 0;
+  if constexpr (Q6) {
+    const uint32_t base = (uint32_t)rel6_step_off(row0, 0), bi = (uint32_t)rel6_block_index(row0, 0);
+    qoff = base + 16 * (2 * bi + (j >> 1)) + 2048 * (j & 1);
+    soff = base + 16 * bi + 8 * (j >> 1);
+    hoff = base + 2 * bi;
+  } else {
+    const uint32_t base = (uint32_t)rel_step_off<DOWN>(row0, 0), ri = c16 & 3;
+    qoff = base + 16 * (uint32_t)rel_piece((int)ri, 0, j);
+    hoff = base + kRelHdr + 16 * ri;
   }
   const rsrc_t wr = make_rsrc(mat, M == kGateUp ? 2 * (size_t)kGateBytes : Q6 ? kDownQ6KBytes : kDownQ4KBytes);
   constexpr int NLOADS = (Q6 ? 5 : 3) * TL;  // weight loads per block
@@ -469,12 +463,12 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
 #pragma unroll
     for (int t = 0; t < TL; ++t) {
       if constexpr (Q6) {
-        const uint32_t st = (uint32_t)rel6_step_off(0, b), bi = (uint32_t)rel6_block_index(0, b);
+        const uint32_t st = (uint32_t)rel6_step_off(0, b) + kTileStep * t, bi = (uint32_t)rel6_block_index(0, b);
         w[t].sc = __builtin_bit_cast(
-            u32x2, __builtin_amdgcn_raw_buffer_load_b64(wr, (int)soff[t], (int)(st + kRel6Sc + 16 * bi), 0));
-        w[t].d = __builtin_amdgcn_raw_buffer_load_b16(wr, (int)hoff[t], (int)(st + kRel6D + 2 * bi), 0);
+            u32x2, __builtin_amdgcn_raw_buffer_load_b64(wr, (int)soff, (int)(st + kRel6Sc + 16 * bi), 0));
+        w[t].d = __builtin_amdgcn_raw_buffer_load_b16(wr, (int)hoff, (int)(st + kRel6D + 2 * bi), 0);
       } else {
-        w[t].hdr = buf_load16<0>(wr, hoff[t], (uint32_t)rel_step_off<DOWN>(0, b) + 64 * (uint32_t)(b & 3));
+        w[t].hdr = buf_load16<0>(wr, hoff, (uint32_t)rel_step_off<DOWN>(0, b) + 64 * (uint32_t)(b & 3) + kTileStep * t);
       }
     }
   };
@@ -483,9 +477,9 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
                            : (uint32_t)rel_step_off<DOWN>(0, b) + 256 * (uint32_t)(b & 3) + kRelQ1 * part;
 #pragma unroll
     for (int t = 0; t < TL; ++t) {
-      (part ? w[t].q1 : w[t].q0) = buf_load16<kNt>(wr, qoff[t], st);
+      (part ? w[t].q1 : w[t].q0) = buf_load16<kNt>(wr, qoff, st + kTileStep * t);
       if constexpr (Q6) {
-        if (part) w[t].qh = buf_load16<kNt>(wr, qoff[t], st - 4096 + kRel6Qh);
+        if (part) w[t].qh = buf_load16<kNt>(wr, qoff, st + kTileStep * t - 4096 + kRel6Qh);
       }
     }
   };
@@ -494,14 +488,14 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   load_q(wa, 0, 0);
   load_q(wa, 0, 1);
   __syncthreads();  // rin, rout
-  // operand row r of plane slot p -> (plane, token); token < 0: a pad row
-  auto row_token = [&](int r, int p, int& plane) {
-    plane = PACK ? (r >= n) + (r >= 2 * n) : p;
-    const int t = PACK ? r - plane * n : r;
+  // operand row r -> (plane, token); token < 0: a pad row
+  auto row_token = [&](int r, int& plane) {
+    plane = P == 1 ? 0 : (r >= n) + (r >= 2 * n);
+    const int t = r - plane * n;
     return t < n ? t : -1;
   };
   // direct-load sources: round k of wave w fills LDS rows 2 (w + 4 k), +1 of
-  // the buffer (row rho = slot * NT16 + r); lane i: row rho0 + i / 32,
+  // the buffer; lane i: row 2 (w + 4 k) + i / 32,
   // slot i % 32 holds piece (i % 32) ^ (r & 7) of that row's block.  The
   // token operand's 16-byte reads (lane (c16, j): row c16, piece
   // (8 j + m) ^ (c16 & 7)) are then free of bank conflicts; an XOR with all
@@ -510,10 +504,9 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   uint32_t src[ROUNDS];
 #pragma unroll
   for (int k = 0; k < ROUNDS; ++k) {
-    const int rho = 2 * (wave + kQWaves * k) + (lane >> 5);
-    const int p = rho / NT16, r = rho - p * NT16;
+    const int r = 2 * (wave + kQWaves * k) + (lane >> 5);
     int plane;
-    const int t = row_token(r, p, plane);
+    const int t = row_token(r, plane);
     uint32_t piece = (uint32_t)((lane & 31) ^ (r & 7));
     // the Q6_K lane's step m = 2 k + u takes elements 128 h + 32 k + 16 s + 8 u:
     // kept at piece 8 j + m of the row too
@@ -554,13 +547,18 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   // weight stream runs one to two blocks ahead on two register sets.
   auto block = [&](int buf, QLane<M> (&w)[TL], const u32x2 (&xsv)[NBX], bool refill, int b) {
     const uint8_t* base = buf ? lds1 : lds0;
+    // the token operand's row c16, piece 8 j + step at step 0
+    uint32_t lane_op = (uint32_t)(c16 * kQRowB + 16 * ((8 * j) ^ (c16 & 7)));
+    // the steps' addresses are made from this one in every block: kept, they
+    // and the 48 accumulators do not fit 168 registers
+    if (TIGHT) asm volatile("" : "+v"(lane_op));
     std::conditional_t<Q6, QScale6, QScale> sc[TL];
 #pragma unroll
     for (int t = 0; t < TL; ++t) {
       // every constant is in a register of its own here: the header's are free
       if constexpr (Q6) {
         sc[t] = qscale6(w[t], j & 1);
-        asm volatile("" : "+v"(sc[t].d), "+v"(sc[t].k[0]), "+v"(sc[t].k[1]), "+v"(sc[t].k[2]), "+v"(sc[t].k[3]));
+        asm volatile("" : "+v"(sc[t].d), "+v"(sc[t].k01), "+v"(sc[t].k23));
       } else {
         sc[t] = qscale(w[t].hdr, sel);
         asm volatile("" : "+v"(sc[t].d), "+v"(sc[t].k), "+v"(sc[t].a), "+v"(sc[t].bc_lo), "+v"(sc[t].bc_hi));
@@ -572,9 +570,10 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
     // Three planes: d C and the min term, which cancels most of its mean, are
     // put together before the running sum, which then holds the result's own
     // partial sums and rounds once per block: 6.0e-7 -> 4.2e-7 of 64 bits for
-    // 16 .. 256 tokens (dot4 4.5e-7), at four additions per tile.  One plane:
-    // the activations' 11 bits set the error (3.4e-4 either way), and the
-    // registers and additions of up to four token blocks cost 5%.
+    // 16 .. 256 tokens (dot4 4.5e-7), at four additions per tile.  Rows without
+    // a min term (planes 1 and 2) take the same two steps wherever they lie.
+    // One plane: the activations' 11 bits set the error (3.4e-4 either way), and
+    // the registers and additions of up to four token blocks cost 5%.
     constexpr bool MIN_FIRST = P == 3 && !Q6;
     auto min_term = [&](int t, int nb, f32x4 a) {
       if constexpr (!Q6) {
@@ -584,7 +583,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
       return a;
     };
     [[maybe_unused]] f32x4 X[TL][NBX];
-    if constexpr (MIN_FIRST) {
+    if constexpr (MIN_FIRST && !TIGHT) {
 #pragma unroll
       for (int t = 0; t < TL; ++t)
 #pragma unroll
@@ -598,37 +597,33 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       const int i0 = 2 * (m & 1);
-      auto operand = [&](int p, int nb, int step) {
-        return *reinterpret_cast<const f16x8*>(base + (p * NT16 + 16 * nb + c16) * kQRowB +
-                                               16 * ((8 * j + step) ^ (c16 & 7)));
+      auto operand = [&](int nb, int step) {
+        return *reinterpret_cast<const f16x8*>(base + 16 * nb * kQRowB + (lane_op ^ (16 * step)));
       };
       if constexpr (Q6) {
-        // a tile's four operands are all 16 registers it takes: one tile at a
-        // time, the token operands held
-        f16x8 alo[PK][NB], ahi[PK][NB];
+        // one nibble of both tiles at a time: the operands are 16 registers
+        auto nibble = [&](auto high) {
+          constexpr bool HIGH = decltype(high)::value;
+          BHalf6 B[TL];
 #pragma unroll
-        for (int p = 0; p < PK; ++p)
+          for (int t = 0; t < TL; ++t) {
+            const u32x4& q = m < 2 ? w[t].q0 : w[t].q1;
+            const f16x2 k = HIGH ? sc[t].k23 : sc[t].k01;
+            B[t] = m < 2 ? build_b6<0, HIGH>(q[i0], q[i0 + 1], w[t].qh[i0], w[t].qh[i0 + 1], k.x)
+                         : build_b6<1, HIGH>(q[i0], q[i0 + 1], w[t].qh[i0], w[t].qh[i0 + 1], k.y);
+          }
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb) alo[p][nb] = operand(p, nb, m), ahi[p][nb] = operand(p, nb, m + 4);
+          for (int nb = 0; nb < NB; ++nb) {
+            const f16x8 a = operand(nb, HIGH ? m + 4 : m);
 #pragma unroll
-        for (int t = 0; t < TL; ++t) {
-          const u32x4& q = m < 2 ? w[t].q0 : w[t].q1;
-          const BPair6 B = m < 2 ? build_b6<0>(q[i0], q[i0 + 1], w[t].qh[i0], w[t].qh[i0 + 1], sc[t].k[0], sc[t].k[2])
-                                 : build_b6<1>(q[i0], q[i0 + 1], w[t].qh[i0], w[t].qh[i0 + 1], sc[t].k[1], sc[t].k[3]);
-          // the weights' rest meets the upper 22 bits of the activations
-          // (2^-11 of a weight times 2^-23 of an activation is left out)
+            for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(a, B[t].r, C[t][nb]);
 #pragma unroll
-          for (int p = PK - 1; p >= 0; --p) {
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-              if (PK == 1 || p < 2) C[t][nb] = mfma_h(alo[p][nb], B.lo_r, C[t][nb]);
-              C[t][nb] = mfma_h(alo[p][nb], B.lo, C[t][nb]);
-              if (PK == 1 || p < 2) C[t][nb] = mfma_h(ahi[p][nb], B.hi_r, C[t][nb]);
-              C[t][nb] = mfma_h(ahi[p][nb], B.hi, C[t][nb]);
-            }
+            for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(a, B[t].v, C[t][nb]);
           }
           __builtin_amdgcn_sched_barrier(0);
-        }
+        };
+        nibble(std::false_type{});
+        nibble(std::true_type{});
       } else {
         BPair B[TL];
 #pragma unroll
@@ -636,17 +631,21 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
           const u32x4& q = m < 2 ? w[t].q0 : w[t].q1;
           B[t] = build_b(q[i0], q[i0 + 1], sc[t].k, sc[t].a);
         }
+        // low nibbles, then high ones
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
+          const f16x8 a = operand(nb, m);
 #pragma unroll
-          for (int p = 0; p < PK; ++p) {
-            const f16x8 alo = operand(p, nb, m), ahi = operand(p, nb, m + 4);
-#pragma unroll
-            for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(alo, B[t].lo, C[t][nb]);
-#pragma unroll
-            for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(ahi, B[t].hi, C[t][nb]);
-          }
+          for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(a, B[t].lo, C[t][nb]);
         }
+        if (TIGHT) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const f16x8 a = operand(nb, m + 4);
+#pragma unroll
+          for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(a, B[t].hi, C[t][nb]);
+        }
+        if (TIGHT) __builtin_amdgcn_sched_barrier(0);
       }
       if (refill && (m & 1)) {
         __builtin_amdgcn_sched_barrier(0);
@@ -654,14 +653,22 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    if constexpr (MIN_FIRST && TIGHT) {
+#pragma unroll
+      for (int t = 0; t < TL; ++t)
+#pragma unroll
+        for (int nb = 0; nb < NBX; ++nb) X[t][nb] = min_term(t, nb, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+    }
 #pragma unroll
     for (int t = 0; t < TL; ++t)
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
         f32x4& a = acc[t][nb];
-        if (MIN_FIRST && nb < NBX) {
+        if (MIN_FIRST) {
+#pragma clang fp contract(off)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) a[i] += fmaf(sc[t].d, C[t][nb][i], X[t][nb][i]);
+          for (int i = 0; i < 4; ++i)
+            a[i] += nb < NBX ? fmaf(sc[t].d, C[t][nb][i], X[t][nb][i]) : sc[t].d * C[t][nb][i];
         } else {
 #pragma unroll
           for (int i = 0; i < 4; ++i) a[i] = fmaf(sc[t].d, C[t][nb][i], a[i]);
@@ -715,16 +722,16 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   auto put = [&](int t, int tile, float gate, float up) {
     const float e = g.xe[rin[t]];
     if (DOWN)
-      g.out[(size_t)rout[t] * kHidden + row[tile]] = gate * e;
+      g.out[(size_t)rout[t] * kHidden + row0 + kTileRows * tile] = gate * e;
     else
-      g.out[(size_t)rout[t] * kFfn + row[tile]] = silu_mul(gate * e, up * e);
+      g.out[(size_t)rout[t] * kFfn + row0 + kTileRows * tile] = silu_mul(gate * e, up * e);
   };
   // gate/up: the up value of a gate lane's row lies two lanes on
   const bool writer = DOWN || (c16 & 2) == 0;
   auto up_of = [](float v) {
     return DOWN ? 0.0f : __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xEE, 0xF, 0xF, false));
   };
-  if constexpr (!PACK) {
+  if constexpr (P == 1) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
@@ -768,10 +775,12 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
 // NB: the largest token block count of a chunk (1 for the 16-token chunks
 // of batched decode, 4 for the 64-token chunks of prefill); a chunk runs the
 // body of the fewest 16-row operand blocks that hold its tokens (three planes:
-// 3 n packed rows up to 10 tokens; from 11 on the packed rows fill three
-// blocks too, and the planes of a token accumulate in registers), so its
-// weight operands are built once for up to 64 tokens and no MFMA runs on an
-// empty block.
+// 3 n rows), so its weight operands are built once for up to 64 tokens and no
+// MFMA runs on an empty block.  (From 11 tokens on three planes fill three
+// blocks however they lie, and letting a token's planes share one accumulator
+// there needs a third of the registers: a step of 256 tokens 1299 against 1322
+// us.  But then a token's bits, and its error, 4.4e-7 against 3.8e-7 of 64
+// bits, depend on how many others chose its expert.)
 // One-dimensional grid: workgroups are handed to the eight XCDs in turn
 // (id % 8), so id -> (xcd = id % 8, k = id / 8).  The items of an expert whose
 // chunks are f .. f + c - 1 are ordered row group by row group, its chunks
@@ -791,18 +800,18 @@ __device__ __forceinline__ void qgemm_chunk(const QGemmArgs& g, uint8_t* lds0, u
                                             int rg) {
   const int n = ck.z;
   if constexpr (P == 3) {
-    if (n <= 5) return qgemm_body<3, 1, 1, true, M, NT>(g, lds0, lds1, rows, ck, rg);
-    if (n <= 10) return qgemm_body<3, 1, 2, true, M, NT>(g, lds0, lds1, rows, ck, rg);
-    return qgemm_body<3, 3, 1, false, M, NT>(g, lds0, lds1, rows, ck, rg);
+    if (n <= 5) return qgemm_body<3, 1, M, NT>(g, lds0, lds1, rows, ck, rg);
+    if (n <= 10) return qgemm_body<3, 2, M, NT>(g, lds0, lds1, rows, ck, rg);
+    return qgemm_body<3, 3, M, NT>(g, lds0, lds1, rows, ck, rg);
   } else {
     if constexpr (NB == 4) {
-      if (n > 48) return qgemm_body<P, P, 4, false, M, NT>(g, lds0, lds1, rows, ck, rg);
-      if (n > 32) return qgemm_body<P, P, 3, false, M, NT>(g, lds0, lds1, rows, ck, rg);
+      if (n > 48) return qgemm_body<P, 4, M, NT>(g, lds0, lds1, rows, ck, rg);
+      if (n > 32) return qgemm_body<P, 3, M, NT>(g, lds0, lds1, rows, ck, rg);
     }
     if constexpr (NB >= 2) {
-      if (n > 16) return qgemm_body<P, P, 2, false, M, NT>(g, lds0, lds1, rows, ck, rg);
+      if (n > 16) return qgemm_body<P, 2, M, NT>(g, lds0, lds1, rows, ck, rg);
     }
-    return qgemm_body<P, P, 1, false, M, NT>(g, lds0, lds1, rows, ck, rg);
+    return qgemm_body<P, 1, M, NT>(g, lds0, lds1, rows, ck, rg);
   }
 }
 

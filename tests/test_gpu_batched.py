@@ -185,6 +185,33 @@ def test_grouped_gemm_chunk_sizes(fdm, oracle, layer, n):
         assert rel_l2(got[t], want) <= 1e-5, t
 
 
+def test_token_bits_do_not_depend_on_the_batch(fdm, layer, batch_kernel):
+    """A token's output bits are the same whatever other tokens share its step,
+    on either path.  Tokens of one routing put every chunk of the grouped GEMMs
+    at n tokens (each operand layout and its edges; 33: 16, 16 and 1), tokens of
+    their own routing mix chunk sizes."""
+    from flash_deepseek_amd.synthetic import make_tokens
+    import torch
+    L, _ = layer
+    K = 8
+
+    def run(X):
+        out = torch.empty_like(X)
+        say(f"moe_forward_batched L={L} T={len(X)} {batch_kernel}")
+        fdm.moe_forward_batched(L, X, None, len(X), K, out)
+        return out
+
+    g = torch.Generator(device="cuda").manual_seed(9)
+    same = torch.randn(7168, generator=g, device="cuda") + \
+        1e-3 * torch.randn(33, 7168, generator=g, device="cuda")
+    mixed = make_tokens(300, 91).view(300, 7168)
+    for X, sizes in ((same, (1, 2, 5, 6, 10, 11, 15, 16, 17)), (mixed, (1, 2, 5, 11, 16, 40, 128))):
+        full = run(X)
+        for n in sizes:
+            assert torch.equal(run(X[:n].contiguous()), full[:n]), n
+        assert torch.equal(run(X[7:29].contiguous()), full[7:29])  # other places in the step
+
+
 @pytest.mark.parametrize("T,K", [(40, 8), (256, 8), (512, 16)])
 def test_grouped_gemm_repeats_bit_exact(fdm, layer, T, K):
     """The same step gives the same bits every time: experts with more than

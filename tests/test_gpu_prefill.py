@@ -243,3 +243,24 @@ def test_prefill_errors(fdm, layers):
         fdm.moe_prefill([L], h, 0, 8, None)
     with pytest.raises(fdm.FdmError):
         fdm.moe_prefill([L], h, 1, 17, None)
+
+
+@pytest.mark.parametrize("q6", [False, True], ids=["q4k_down", "q6k_down"])
+def test_prefill_bits_do_not_depend_on_the_prompt(fdm, layers, q6):
+    """A token's bits are the same whatever other tokens of the prompt are run
+    with it, so a prompt may be cut anywhere."""
+    import torch
+    from flash_deepseek_amd.synthetic import make_tokens
+    L, lay = next(x for x in layers if bool(x[1].down_q6) == q6)
+    X = make_tokens(300, 95).view(300, 7168)
+    norm = to_dev(np.ones(7168, np.float32))
+
+    def run(x):
+        h = x.clone()
+        say(f"moe_prefill L={L} T={len(h)}")
+        fdm.moe_prefill([L], h, len(h), 8, [norm])
+        return h
+
+    full = run(X)
+    for a, b in ((0, 1), (0, 16), (16, 40), (40, 150), (150, 300)):
+        assert torch.equal(run(X[a:b]), full[a:b]), (a, b)
