@@ -149,6 +149,53 @@ def test_batched_fp32_grade(fdm, oracle, layer, batch_kernel, T, kind):
         assert m_got <= 4 * m_f32, (t, m_got, m_f32)
 
 
+@pytest.mark.parametrize("q6", [False, True], ids=["q4k_down", "q6k_down"])
+def test_grouped_gemms_no_further_off_than_dot4(fdm, oracle, q6):
+    """Small steps run the grouped GEMMs by default, so these may be no further
+    from float64 than the dot4 kernels, on weights around zero (the min term
+    takes back most of what the quants sum to).  They carry more bits of the
+    activations (33 against 24) and no sum of theirs is less exact, hence 0.9:
+    the scatter of the ratio over 5 x 7168 outputs is a few percent."""
+    import torch
+    from flash_deepseek_amd.synthetic import make_layer
+    L, T, K, gate = 16, 5, 8, 57344 * 144
+    say(f"building layer L={L} around zero, down_q6={q6}")
+    lay = make_layer(2050, down_q6=q6)
+    g = torch.Generator(device="cuda").manual_seed(3)
+
+    def scales(shape, unit):
+        return ((torch.rand(shape, generator=g, device="cuda") + 0.5) * unit).half()
+
+    for e in (lay.experts.view(256, -1), lay.shared.view(1, -1)):
+        q4 = e[:, :(2 if q6 else 3) * gate].view(len(e), -1, 144)
+        d = scales(q4.shape[:2], 8e-5)
+        q4[..., :4] = torch.stack([d, (d.float() * 7.5).half()], -1).view(torch.uint8)
+        if q6:
+            down = e[:, 2 * gate:].view(len(e), -1, 210)
+            down[..., 208:] = scales(down.shape[:2] + (1,), 1.5e-5).view(torch.uint8)
+    fdm.attach_layer(L, lay.experts, lay.expert_size, lay.Wg, lay.bias, lay.shared)
+    try:
+        X = np.random.default_rng(21).standard_normal((T, 7168)).astype(np.float32)
+        got, dX = {}, to_dev(X.ravel())
+        idx, w = torch.empty(T * K, dtype=torch.int32, device="cuda"), empty_f32(T * K)
+        for mode in (fdm.BATCH_DOT4, fdm.BATCH_MFMA):
+            prev = fdm.set_batch_kernel(mode)
+            out = empty_f32(T * 7168)
+            say(f"moe_forward_batched L={L} T={T} mode {mode}")
+            fdm.moe_forward_batched(L, dX, None, T, K, out, idx, w)
+            fdm.set_batch_kernel(prev)
+            got[mode] = to_host(out).reshape(T, 7168)
+    finally:
+        fdm.release_layer(L)
+    gi, gw = to_host(idx).reshape(T, K), to_host(w).reshape(T, K)
+    want = np.stack([np.float64(oracle.expert_ffn(lay.expert_bytes(-1), q6, X[t])) +
+                     sum(np.float64(gw[t][k]) * oracle.expert_ffn(lay.expert_bytes(int(gi[t][k])), q6, X[t])
+                         for k in range(K)) for t in range(T)])
+    dot4, mfma = (rel_l2(got[m], want) for m in (fdm.BATCH_DOT4, fdm.BATCH_MFMA))
+    print(f"q6={q6}: dot4 {dot4:.3e}, grouped GEMMs {mfma:.3e} of float64")
+    assert mfma <= 0.9 * dot4
+
+
 @pytest.mark.parametrize("n", [1, 5, 6, 10, 11, 16, 17, 22, 27, 32, 33])
 def test_grouped_gemm_chunk_sizes(fdm, oracle, layer, n):
     """n tokens that all choose the same experts, so every chunk of the
