@@ -410,7 +410,6 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
   constexpr int NBLK = KD / kQK;             // 8 or 28 (even)
   constexpr int NT16 = 16 * NB;              // operand rows
   constexpr int NTOK = NT16 / P;
-  constexpr bool TIGHT = P == 3 && NB == 3;  // registers are short
   constexpr int NBX = (NTOK + 15) / 16;      // 16-row blocks that hold plane 0 rows
   constexpr int ROUNDS = NT16 / (2 * kQWaves);  // direct loads per wave per block (2 rows each)
   static_assert(ROUNDS * 2 * kQWaves == NT16, "the direct loads tile the buffer");
@@ -551,7 +550,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
     uint32_t lane_op = (uint32_t)(c16 * kQRowB + 16 * ((8 * j) ^ (c16 & 7)));
     // the steps' addresses are made from this one in every block: kept, they
     // and the 48 accumulators do not fit 168 registers
-    if (TIGHT) asm volatile("" : "+v"(lane_op));
+    if (P == 3 && NB == 3) asm volatile("" : "+v"(lane_op));
     std::conditional_t<Q6, QScale6, QScale> sc[TL];
 #pragma unroll
     for (int t = 0; t < TL; ++t) {
@@ -583,7 +582,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
       return a;
     };
     [[maybe_unused]] f32x4 X[TL][NBX];
-    if constexpr (MIN_FIRST && !TIGHT) {
+    if constexpr (MIN_FIRST) {
 #pragma unroll
       for (int t = 0; t < TL; ++t)
 #pragma unroll
@@ -631,33 +630,24 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
           const u32x4& q = m < 2 ? w[t].q0 : w[t].q1;
           B[t] = build_b(q[i0], q[i0 + 1], sc[t].k, sc[t].a);
         }
-        // low nibbles, then high ones
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
           const f16x8 a = operand(nb, m);
 #pragma unroll
           for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(a, B[t].lo, C[t][nb]);
         }
-        if (TIGHT) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
           const f16x8 a = operand(nb, m + 4);
 #pragma unroll
           for (int t = 0; t < TL; ++t) C[t][nb] = mfma_h(a, B[t].hi, C[t][nb]);
         }
-        if (TIGHT) __builtin_amdgcn_sched_barrier(0);
       }
       if (refill && (m & 1)) {
         __builtin_amdgcn_sched_barrier(0);
         load_q(w, b + 2, m >> 1);
         __builtin_amdgcn_sched_barrier(0);
       }
-    }
-    if constexpr (MIN_FIRST && TIGHT) {
-#pragma unroll
-      for (int t = 0; t < TL; ++t)
-#pragma unroll
-        for (int nb = 0; nb < NBX; ++nb) X[t][nb] = min_term(t, nb, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
     }
 #pragma unroll
     for (int t = 0; t < TL; ++t)
