@@ -2,9 +2,9 @@
 fixed device scratch (it allocates nothing), against fdm_moe_forward_batched
 on the same inputs.  Both run the same kernels on buffers of the same
 shapes, so the outputs, the routing and the distinct-expert count must be
-bit-identical.  Two no-allocation calls run back to back, the second with
-fewer tokens (and on the digit-kernel path, T < FDM_BATCH_MFMA_MIN_T), so
-a leftover of the first call in the shared scratch would show; sizes past
+bit-identical.  No-allocation calls run back to back with fewer and fewer
+tokens (the last on the digit kernels, T < FDM_BATCH_MFMA_MIN_T), so
+a leftover of an earlier call in the shared scratch would show; sizes past
 the scratch's limits are rejected.  That the call allocates nothing is
 checked by capturing it into a HIP graph on a fresh stream in global
 capture mode, where any allocation (a workspace for that stream included)
@@ -46,14 +46,28 @@ def step(fdm, fn, L, X, H, T):
     return out, idx, w, nd
 
 
-@pytest.mark.parametrize("T", [16, 3], ids=["mfma_path", "dot4_path"])
-def test_noalloc_captures_in_a_graph(fdm, layer, T):
+@pytest.fixture
+def path(request, fdm):
+    """The expert path of the test: what AUTO takes at its T, or dot4 forced."""
+    if request.param == "dot4_forced":
+        prev = fdm.set_batch_kernel(fdm.BATCH_DOT4)
+        yield request.param
+        fdm.set_batch_kernel(prev)
+    else:
+        yield request.param
+
+
+@pytest.mark.parametrize("T,path", [(16, "mfma"), (3, "mfma"), (1, "dot4"), (32, "dot4_forced")],
+                         indirect=["path"])
+def test_noalloc_captures_in_a_graph(fdm, layer, T, path):
     """The property the entry point exists for: it allocates nothing.  The
     call is captured into a HIP graph on a fresh stream in global capture
     mode (hipMalloc, and so a stream workspace, is refused there and the
     capture fails).  Each replay, with eager work and synchronisations
     between replays, equals the eager fdm_moe_forward_batched bit for bit."""
     import torch
+    if path != "dot4_forced":  # AUTO takes the path that the test is named for
+        assert path == ("mfma" if T >= fdm.BATCH_MFMA_MIN_T else "dot4")
     L = layer
     X, H = tokens(T, 43 + T)
     say(f"moe_forward_batched (eager reference) L={L} T={T}")
@@ -90,7 +104,9 @@ def test_noalloc_captures_in_a_graph(fdm, layer, T):
 
 def test_noalloc_matches_batched(fdm, layer):
     L = layer
-    cases = [(fdm.NOALLOC_MAX_T, 31), (5, 37)]  # the largest step, then a smaller one
+    # the largest step, a smaller one, and one on the digit kernels
+    cases = [(fdm.NOALLOC_MAX_T, 31), (5, 37), (1, 39)]
+    assert cases[-1][0] < fdm.BATCH_MFMA_MIN_T <= cases[-2][0]
     inputs = [tokens(T, seed) for T, seed in cases]
     got = []
     for (T, _), (X, H) in zip(cases, inputs):
