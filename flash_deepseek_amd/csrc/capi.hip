@@ -1507,8 +1507,9 @@ QScratch workspace_q(const Workspace& w) {
 
 // The expert half of one step on the grouped GEMMs, on the planes of the
 // token rows that the caller has written: dispatch with the chunk list,
-// gate/up + SwiGLU into b.act, the planes of b.act and the down into b.eo.  A Q6_K down takes three planes always, in chunks of their
-// size (one-plane callers have a second chunk list for it in the workspace).
+// gate/up + SwiGLU into b.act, the planes of b.act and the down into b.eo.  A
+// Q6_K down takes three planes always, in chunks of their size (one-plane
+// callers have a second chunk list for it in the workspace).
 int run_qgemm_experts(const Layer* y, const BatchArgs& b0, int planes, const QScratch& w, hipStream_t s) {
   BatchArgs b = b0;
   const int T = b.T, K = b.K;
@@ -1608,7 +1609,6 @@ int fdm_moe_prefill(const int* layers, int n_layers, float* d_H, int T, int K,
     b.idx = idx;
     b.w = w.w;
     b.act = w.b_act;
-    b.act_xd = w.b_act_xd;
     b.eo = w.b_eo;
     b.seg_start = w.b_seg;
     b.pair_tok = w.b_pair_tok;

@@ -302,7 +302,8 @@ int fdm_set_layer_spin_limit(unsigned polls, unsigned *prev);
  * are read once per step (config 3; the reference decodes one token at a
  * time, infer.m:2219-2229).  Per token t the result is fdm_moe_layer's:
  *   hidden[t] = h_in[t] + sum_k w[t][k] E_k(h_post[t]) + S(h_post[t])
- * with route() per token (bit-exact idx / w).  d_X, d_H_in, d_hidden:
+ * with route() per token (bit-exact idx / w); token t's bits do not depend on
+ * the other tokens of the step.  d_X, d_H_in, d_hidden:
  * [T][7168] fp32 (d_H_in may be NULL).  d_idx / d_w ([T][K], optional)
  * receive the routing; d_n_distinct (optional, device int) the number of
  * distinct routed experts of the step.  1 <= T <= FDM_MAX_TOKENS. */
@@ -351,10 +352,11 @@ int fdm_rms_norm(const float *d_x, const float *d_w, float *d_o, int T, int d, v
 /* ---- prefill: T tokens through n_layers resident MoE layers,
  *   h <- h + MoE_l(rms_norm(h, norm_w[l]))   for l = 0 .. n_layers-1
  * (infer.m:1850, 1878-1922), in place on d_H [T][7168] fp32.  Routing is
- * route() per token on the fp32 rms_norm output (bit-exact); the Q4_K
- * expert GEMMs run on MFMA with fp32 accumulation, the weights as the exact
- * integers 1024 + sc*q in fp16 and the activations as one fp16 plane (a Q6_K
- * down runs on the digit kernels).  layers / d_norm_w: host arrays of
+ * route() per token on the fp32 rms_norm output (bit-exact); the expert
+ * GEMMs run on MFMA with fp32 accumulation, Q4_K weights as the exact
+ * integers sc*q in fp16 against one fp16 plane of the activations, a Q6_K
+ * down's sc*(q - 32) as two fp16 values against three.  A token's bits do not
+ * depend on the other tokens of the call.  layers / d_norm_w: host arrays of
  * n_layers layer ids / device pointers to [7168] fp32.  d_idx (optional,
  * [n_layers][T][K]) receives every layer's routing.  1 <= T <= FDM_MAX_TOKENS. */
 int fdm_moe_prefill(const int *layers, int n_layers, float *d_H, int T, int K,
