@@ -1647,6 +1647,8 @@ struct BatchScratch {
 // into one MFMA operand they take 96 against 102 us at 2 tokens, 154 / 187 at
 // 5, 199 / 275 at 8 and 264 / 376 at 12 (K = 8, Q4_K down; Q6_K 112 / 114,
 // 180 / 217, 235 / 325, 305 / 449; K = 4 and 16 alike), and 79 / 69 at one.
+// They are also closer to 64 bits: 2.9 .. 3.0e-7 at 2 to 256 tokens against 3.9
+// .. 5.2e-7 (Q6_K down 2.7 .. 2.8e-7 against 3.4 .. 3.8e-7).
 bool batch_uses_mfma(int T) {
   return g_batch_mode == FDM_BATCH_MFMA || (g_batch_mode == FDM_BATCH_AUTO && T >= FDM_BATCH_MFMA_MIN_T);
 }

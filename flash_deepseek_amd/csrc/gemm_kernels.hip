@@ -24,8 +24,7 @@
 // two: the largest |x'| lies in [2^13, 2^14)): P = 3 carries every fp32
 // value exactly (hi + mid + lo, 33 significant bits) -- batched decode and
 // every Q6_K down, fp32 grade; P = 1 carries 11 bits -- prefill, whose bar is
-// 1e-2.  X_sb is the
-// fp32 sum of the planes' values.
+// 1e-2.  X_sb is the sum of the planes' values (planes_device.h).
 //
 // Mapping.  A workgroup of 4 waves owns 64 gate and 64 up rows (wave w:
 // rows 16 w .. 16 w + 15 of both, two of gate and the same two of up by turns
@@ -43,34 +42,36 @@
 // b + 1 streams in while block b is contracted.
 //
 // What bounds it.  A read of the same weight lines with the same tiles and
-// no math takes 180-205 us for 71 experts' gate and up (5.7-6.6 TB/s); the
-// vector ALU (about 95 instructions per 16-row tile and block, 9 per 8
-// weights for the operand) and the matrix cores (16 cycles per 16x16x32, 32
-// per 16x16x4) need about as long and overlap only partly, so the kernel
-// lives on loads in flight and on few instructions:
+// no math takes 180-205 us for 71 experts' gate and up (5.7-6.6 TB/s).  The
+// vector ALU (three planes: 97, 105 and 117 instructions per 16-row tile and
+// block at up to 5, 10 and 16 tokens, of them 64 for the weight operands; one
+// plane 93 .. 105) and the matrix cores (8, 16 or 24 16x16x32 of 16 cycles and
+// two 16x16x4 of 32) need about as long and overlap only partly, so the kernel
+// lives on loads in flight and on few instructions.  What that came to, gate/up
+// of a step of 16 tokens unless said otherwise, each before and after on one box
+// (boxes differ by 5%):
 //  - the three planes of a chunk of few tokens share 16-row operands:
 //    up to 5 tokens cost 8 MFMAs per tile and block instead of 24 and a
 //    third of the LDS traffic; with that, two tiles per wave and three waves
-//    per SIMD beat four tiles and two waves (16-token step 234 against 279 us);
+//    per SIMD beat four tiles and two waves (328 -> 234 us; four tiles 279);
 //  - each weight register is refilled with block b + 2 right after its last
-//    use, so the stream runs one to two blocks ahead on two register sets
-//    (234 -> 219 us, 64 tokens 479 -> 443 us);
-//  - buffer loads: no address arithmetic on the vector ALU, and a pad row's
+//    use, so the stream runs one to two blocks ahead on two register sets; and
+//    buffer loads: no address arithmetic on the vector ALU, and a pad row's
 //    planes and sub-block sums lie past the buffer's end, so they cost no
-//    traffic (and the sums no select that waits for the load);
-//  - a block's scales and mins are taken from the header two at a time
-//    (105 -> 95 instructions; 213, 467 and 910 us in the figures below);
+//    traffic and the sums no select that waits for the load (234 -> 219);
+//  - a block's scales and mins are taken from the header two at a time (220 ->
+//    213);
+//  - three planes' items lie on the XCDs in contiguous ranges (221 -> 210);
 //  - the resident layout's row-fastest pieces halve the L1 cycles of a weight
-//    load (16 / 64 / 256 tokens 210 -> 199, 468 -> 444, 883 -> 855 us);
+//    load (210 -> 199; 64 / 256 tokens 468 -> 444, 883 -> 855);
 //  - an expert with one chunk is streamed past the L2 (nontemporal).
-// gate/up of 71 / 132 / 188 experts (16 / 64 / 256 tokens): 328 -> 219, 587 ->
-// 443, 1032 -> 925 us; the down of 16 / 256 tokens 151 -> 122, 517 -> 479 us;
-// one plane, 512 tokens: gate/up 994 -> 906, down 522 -> 499 us.
-// The Q6_K down costs about 200 vector instructions per tile and block (two
-// halves per weight, six bits from two places) and 16 .. 40 MFMAs, and still
-// takes 383 us where the dot4 kernel, which unpacks every weight again for
-// every token, took 922 (132 experts of 64 tokens); 522 against 1906 us for
-// 150 prompt tokens.
+// On one build and box: gate/up of 71 / 130 / 176 experts (16 / 64 / 256 tokens)
+// 213, 459 and 909 us, the down of 16 / 256 tokens 117 and 486 us; one plane, 512
+// tokens, gate/up 844, down 474 us.
+// The Q6_K down costs 196 .. 208 vector instructions per tile and block (two
+// halves per weight, six bits from two places) and 16, 32 or 48 MFMAs: 375 us for
+// 130 experts of 64 tokens, where the dot4 kernel, which unpacks every weight
+// again for every token, took 922; 538 against 1906 us for 150 prompt tokens.
 #include "fdm_internal.h"
 #include "planes_device.h"
 #include "route_device.h"
@@ -568,8 +569,9 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& g, uint8_t* lds0, ui
     __builtin_amdgcn_sched_barrier(0);
     // Three planes: d C and the min term, which cancels most of its mean, are
     // put together before the running sum, which then holds the result's own
-    // partial sums and rounds once per block: 6.0e-7 -> 4.2e-7 of 64 bits for
-    // 16 .. 256 tokens (dot4 4.5e-7), at four additions per tile.  Rows without
+    // partial sums and rounds once per block (6.0e-7 -> 4.2e-7 of 64 bits for
+    // 16 .. 256 tokens; 2.9e-7 with the planes' sums in 64 bits and each plane
+    // summed by itself; dot4 4.5e-7), at four additions per tile.  Rows without
     // a min term (planes 1 and 2) take the same two steps wherever they lie.
     // One plane: the activations' 11 bits set the error (3.4e-4 either way), and
     // the registers and additions of up to four token blocks cost 5%.
